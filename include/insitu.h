@@ -296,9 +296,13 @@ enum {
                                         attend elsewhere), 1 the scan attend, 2 the chunked attend
                                         (the decode step too), 3 the decode step's own kernel;
                                         INSITU_EINVAL if the kernel does not handle the cache   */
-    INSITU_DEBUG_APPEND = 5          /* the append's kernel: 0 automatic (lane = row where it
+    INSITU_DEBUG_APPEND = 5,         /* the append's kernel: 0 automatic (lane = row where it
                                         handles the format: d = 64, 4/2- or 2/2-bit codes), 1 the
                                         lane-per-channel kernel for every format                */
+    INSITU_DEBUG_PREFILL = 6         /* the causal attends' kernel: 0 automatic (the prefill kernel
+                                        where it handles the format and the queries fill it), 1 the
+                                        decode attends over a virtual batch, 2 the prefill kernel;
+                                        INSITU_EINVAL if it does not handle the cache            */
 };
 int insitu_cache_debug(insitu_cache *cache, int32_t what, int64_t value);
 /* The statistics the cache's kernels have gathered since they were last cleared (an

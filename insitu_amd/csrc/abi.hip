@@ -191,6 +191,7 @@ struct insitu_cache {
     int64_t *prefill_len = nullptr;
     int32_t spin_limit = 1 << 20;         // insitu_cache_debug
     int32_t path = 0;                     // insitu_cache_debug: 0 auto, 1 scan, 2 chunked, 3 step kernel
+    int32_t prefill_path = 0;             // insitu_cache_debug: 0 auto, 1 virtual batch, 2 prefill kernel
     int32_t append_path = 0;              // insitu_cache_debug: 0 auto, 1 the lane-per-channel kernel
 };
 
@@ -821,6 +822,36 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 
 }  // namespace
 
+// Whether a causal attend runs on the prefill kernel (attend_prefill.hip). Its waves walk their
+// rows' whole contexts, so a grid that does not fill the chip takes a time of its own in the
+// context's length alone; the chunked attend over a virtual batch spreads one query's context over
+// the chip and takes time in proportion to the queries. Fitted to both, measured over 1 to 256
+// queries and 128 to 32,768 rows (us, 32 query heads; e.g. 16 queries of 2,048 rows at d = 64:
+// 214 here, 68 there; 128: 218 and 275; 256 of 32,768: 2,514 and 7,106).
+static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
+    if (mode == INSITU_SERIAL || !prefill_supported(gv) || k->prefill_path == 1) return false;
+    if (k->prefill_path == 2) return true;
+    if (k->path != 0) return false;
+    if (!k->chunked) return true;           // else token by token
+    const bool two = mode == INSITU_TWO_PASS, d64 = gv.d == 64;
+    const double t = (double)(base + n_q);
+    const double here = (two ? 14.0 : 20.0) + t * (d64 ? 0.075 : 0.16) * (two ? 1.2 : 1.0);
+    const double there = (d64 ? 28.0 : 40.0) + 25.0 * (t < 1500.0 ? t / 1500.0 : 1.0) +
+                         t * (double)n_q * gv.n_q * (d64 ? 2.65e-5 : 5.2e-5) * (two ? 1.95 : 1.0);
+    return here < there;
+}
+
+static int prefill_kernel_launch(insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, const int32_t *q,
+                                 int32_t *out, int32_t mode, bool timed = true) {
+    LaunchEv ev;
+    int rc = timed ? timing_events(k->ctx, &ev) : INSITU_OK;
+    if (rc) return rc;
+    HIP_TRY(launch_attend_prefill(k->ctx->stream, gv, k->tabs, q, out, base, n_q, mode == INSITU_TWO_PASS ? 1 : 0, ev,
+                                  k->stats),
+            "prefill attend launch");
+    return INSITU_OK;
+}
+
 // The prefill launches over a scratch the caller provides (scr, lengths len_dev for
 // PREFILL_QB queries); shared by insitu_attend_causal and its allocation-free variant.
 static int prefill_launches(insitu_cache *k, const Geom &gv, const PrefillPlan &pl, ChunkScratch &scr,
@@ -881,6 +912,10 @@ static int causal_impl(insitu_cache *k, const Geom &gv, int64_t base, int64_t n_
     int rc = stats ? zero_stats(k) : INSITU_OK;
     if (rc) return rc;
     if (n_q == 0) return copy_stats(k, stats);
+    if (use_prefill_kernel(k, gv, base, n_q, mode)) {
+        rc = prefill_kernel_launch(k, gv, base, n_q, q, out, mode);
+        return rc ? rc : copy_stats(k, stats);
+    }
     const PrefillPlan pl = prefill_plan(*k->api, chunk_geom(k, gv), base, n_q, PREFILL_SCRATCH_BUDGET);
     if (!k->prefill_len) HIP_TRY(hipMalloc(&k->prefill_len, PREFILL_QB * sizeof(int64_t)), "hipMalloc");
     if (mode != INSITU_SERIAL && k->chunked && k->prefill_scr.bytes < pl.bytes) {
@@ -951,6 +986,7 @@ int insitu_attend_causal_static(insitu_cache *k, int32_t seq, int64_t base, int6
             return fail(INSITU_EBADLEN, buf);
         }
     }
+    if (use_prefill_kernel(k, gv, base, n_q, mode)) return prefill_kernel_launch(k, gv, base, n_q, q, out, mode, false);
     return prefill_launches(k, gv, pl, ss.cs, ss.len, base, n_q, q, out, mode, false);
 }
 
@@ -1060,6 +1096,11 @@ int insitu_cache_debug(insitu_cache *k, int32_t what, int64_t value) {
         if (value < 0 || value > 3)
             return fail(INSITU_EINVAL, "path is 0 (auto), 1 (scan), 2 (chunked) or 3 (step kernel)");
         k->path = (int32_t)value;
+        return INSITU_OK;
+    case INSITU_DEBUG_PREFILL:
+        if (value < 0 || value > 2) return fail(INSITU_EINVAL, "prefill is 0 (auto), 1 (virtual batch) or 2 (prefill kernel)");
+        if (value == 2 && !prefill_supported(k->g)) return fail(INSITU_EINVAL, "the prefill kernel does not handle this cache");
+        k->prefill_path = (int32_t)value;
         return INSITU_OK;
     case INSITU_DEBUG_APPEND:
         if (value < 0 || value > 1) return fail(INSITU_EINVAL, "append kernel is 0 (auto) or 1 (lane per channel)");

@@ -319,6 +319,11 @@ hipError_t launch_step_write(hipStream_t s, const Geom &g, const Tables *t, cons
                              const int32_t *kw, const int32_t *vw, int rounds,
                              const uint64_t (*signs)[2], int32_t *qr, double *qd, int32_t *qok,
                              const int64_t *len_in, int64_t *len_out, DevStats *st);
+// The prefill attend on matrix cores (attend_prefill.hip): query i of n_q (rows of q, (n_q,
+// g.n_q, d)) over rows 0 .. base + i of the sequence at g.base; no scratch, one launch.
+bool prefill_supported(const Geom &g);
+hipError_t launch_attend_prefill(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,
+                                 int64_t base, int64_t n_q, int two_pass, LaunchEv ev, DevStats *st);
 hipError_t launch_attend_serial(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q,
                                 int32_t *out, const int64_t *len, int two_pass, LaunchEv ev,
                                 DevStats *st);
