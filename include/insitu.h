@@ -294,7 +294,9 @@ enum {
                                         decode step on its own kernel where it handles the cache,
                                         the chunked attend where it handles the cache, the scan
                                         attend elsewhere), 1 the scan attend, 2 the chunked attend
-                                        (the decode step too), 3 the decode step's own kernel;
+                                        (the decode step too), 3 the decode step's own kernel,
+                                        4 two-pass mode's split attend
+                                        (any other mode automatic);
                                         INSITU_EINVAL if the kernel does not handle the cache   */
     INSITU_DEBUG_APPEND = 5,         /* the append's kernel: 0 automatic (lane = row where it
                                         handles the format: d = 64, 4/2- or 2/2-bit codes), 1 the

@@ -17,7 +17,7 @@ SEQUENTIAL, TWO_PASS, SPLIT, SERIAL = range(4)
 DEBUG_DECODE_CALLS, DEBUG_PREFILL_CALLS, DEBUG_SPIN_LIMIT, DEBUG_PATH, DEBUG_APPEND = 1, 2, 3, 4, 5
 DEBUG_PREFILL = 6
 PREFILL_AUTO, PREFILL_BATCH, PREFILL_MATRIX = 0, 1, 2
-PATH_AUTO, PATH_SCAN, PATH_CHUNKED, PATH_STEP = 0, 1, 2, 3
+PATH_AUTO, PATH_SCAN, PATH_CHUNKED, PATH_STEP, PATH_SPLIT = 0, 1, 2, 3, 4
 MODES = {"online": SEQUENTIAL, "sequential": SEQUENTIAL, "two_pass": TWO_PASS,
          "split": SPLIT, "serial": SERIAL}
 

@@ -181,6 +181,7 @@ struct insitu_cache {
     bool vsplit = false;                  // ... seeing each KV head's 8 query heads as two chains of 4
     bool gpad = false;                    // ... computing fewer than 4 query heads a KV head in 4 slots
     bool scan = false;                    // the scan attend does (sequential mode)
+    bool split = false;                   // the split attend does (two-pass mode)
     bool step = false;                    // the fused step's own kernel does (sequential mode)
     int64_t step_mc = 0;                  // its layout: chunks per sequence
     ChunkScratch scr;                     // decode attends: run sums and counters, one call's worth
@@ -190,7 +191,7 @@ struct insitu_cache {
     ChunkScratch prefill_scr;
     int64_t *prefill_len = nullptr;
     int32_t spin_limit = 1 << 20;         // insitu_cache_debug
-    int32_t path = 0;                     // insitu_cache_debug: 0 auto, 1 scan, 2 chunked, 3 step kernel
+    int32_t path = 0;                     // insitu_cache_debug: 0 auto, 1 scan, 2 chunked, 3 step kernel, 4 split
     int32_t prefill_path = 0;             // insitu_cache_debug: 0 auto, 1 virtual batch, 2 prefill kernel
     int32_t append_path = 0;              // insitu_cache_debug: 0 auto, 1 the lane-per-channel kernel
 };
@@ -551,11 +552,13 @@ int insitu_cache_create(insitu_ctx *c, const insitu_cache_desc *desc, insitu_cac
         k->chunked = k->api->supported(chunk_geom(k, g), desc->capacity);
         k->gpad = k->chunked;
     }
-    if (e == hipSuccess && (k->chunked || k->scan || k->step)) {
-        size_t nb = 0;
+    k->split = split_supported(g, desc->capacity);
+    if (e == hipSuccess && (k->chunked || k->scan || k->step || k->split)) {
+        size_t nb = k->split ? split_scratch_bytes(g, desc->capacity) : 0;
         if (k->step) {
             k->step_mc = step_max_chunks(desc->capacity);
-            nb = step_scratch_bytes(g, k->step_mc);
+            const size_t nk = step_scratch_bytes(g, k->step_mc);
+            nb = nk > nb ? nk : nb;
         }
         if (k->chunked) {
             k->max_chunks = k->api->max_chunks(desc->capacity);
@@ -710,7 +713,36 @@ static bool use_scan(const insitu_cache *k, int32_t mode) {
 // 512 chunks of 1,024 tokens); the test hook can pin the chunked (2) or scan (1) attend.
 static bool use_step_kernel(const insitu_cache *k, int32_t mode) {
     if ((mode != INSITU_SEQUENTIAL && mode != INSITU_SPLIT) || !k->step) return false;
-    return k->path == 0 || k->path == 3;
+    return k->path != 1 && k->path != 2;
+}
+
+// The split attend: pinned (4), or automatically in two-pass mode, where the chunked attend scores
+// every token in a first launch and has each chunk's workgroup do so again. (Its workgroups wait on
+// nobody: a cache whose waits are under test keeps the kernels that wait.) Measured, call to call,
+// chunked / split us at tokens x batch, first a flat softmax, then one where a few tokens have all
+// the weight (every other token is then skipped by both, and fixed costs show):
+//   d = 64, 4-bit keys, 2-bit values, 4 query heads a KV head, 8 KV heads:
+//     16 x 1: 49/42, 49/41   2,048 x 1: 91/44, 55/43   32,768 x 1: 97/59, 62/49   131,072 x 1: 281/98, 147/64
+//     100 x 16: 54/46, 53/45   8,192 x 16: 259/84, 114/63   32,768 x 16: 833/213, 356/109
+//   8 query heads a KV head, 4 KV heads, 3-bit keys:
+//     16 x 1: 49/44, 49/43   2,048 x 1: 89/49, 54/48   131,072 x 1: 237/98, 143/63   131,072 x 16: 2,904/484, 1,509/206
+//   d = 128, 4-bit keys, 2-bit values, 8 KV heads:
+//     16 x 1: 57/43, 57/42   2,048 x 1: 125/48, 64/46   131,072 x 1: 414/130, 163/82   32,768 x 16: 1,440/263, 462/150
+//   d = 128, 3-bit keys and values (a lane's key codes are three words of two planes):
+//     16 x 1: 57/45, 58/45   2,048 x 1: 135/57, 65/56   8,192 x 1: 136/77, 66/71   131,072 x 1: 462/157, 170/97
+//     512 x 16: 95/71, 62/71   4,097 x 16: 237/113, 99/97   32,768 x 16: 1,578/330, 482/163
+// so it is taken everywhere but in the last format between the sizes where it was slower on peaked
+// weights.
+static bool use_split(const insitu_cache *k, int32_t mode, bool step) {
+    if (mode != INSITU_TWO_PASS || !k->split) return false;
+    if (k->path == 4) return true;
+    if (k->path != 0 || k->spin_limit == 0) return false;
+    const Geom &g = k->g;
+    if (g.d == 64 || g.kb != 3) return true;
+    int64_t longest = 0;
+    for (int64_t n : k->len_host) longest = n > longest ? n : longest;
+    const int64_t rows = (int64_t)g.batch * g.n_kv * (longest + (step ? 1 : 0));
+    return rows <= (1 << 15) || rows >= (1 << 19);
 }
 
 // q_staged: the chunked path's fp64 query staging already holds q (the step's
@@ -724,6 +756,14 @@ static int attend_impl(insitu_cache *k, const int32_t *q, int32_t *out, int32_t 
     LaunchEv ev;
     int rc = timing_events(k->ctx, &ev);
     if (rc) return rc;
+    if (use_split(k, mode, step != nullptr)) {
+        int64_t longest = 0;
+        for (int64_t n : k->len_host) longest = n > longest ? n : longest;
+        HIP_TRY(launch_attend_split(k->ctx->stream, k->g, k->tabs, q, out, len, k->scr, longest + (step ? 1 : 0), step, ev,
+                                    k->stats),
+                "split attend launch");
+        return INSITU_OK;
+    }
     if (use_scan(k, mode)) {
         // the scan attend, its grid sized by the longest sequence
         if (!ep) HIP_TRY(scratch_begin(k->ctx->stream, k->scr, &ep), "scratch clear");
@@ -831,7 +871,7 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
     if (mode == INSITU_SERIAL || !prefill_supported(gv) || k->prefill_path == 1) return false;
     if (k->prefill_path == 2) return true;
-    if (k->path != 0) return false;
+    if (k->path != 0 && k->path != 4) return false;
     if (!k->chunked) return true;           // else token by token
     const bool two = mode == INSITU_TWO_PASS, d64 = gv.d == 64;
     const double t = (double)(base + n_q);
@@ -1010,11 +1050,11 @@ int insitu_step(insitu_cache *k, const int32_t *q, const int32_t *kw, const int3
     // token attends to itself), then the attend (:337-345). In chunked
     // sequential mode at d = 64 that is one launch; otherwise one write kernel
     // (which also stages the rotated queries for a chunked attend) and the attend.
-    const bool scan = use_scan(k, mode);
-    const bool chunked = !scan && mode != INSITU_SERIAL && k->chunked;
+    const bool split = use_split(k, mode, true), scan = !split && use_scan(k, mode);
+    const bool chunked = !split && !scan && mode != INSITU_SERIAL && k->chunked;
     // (a KV head seen as two chains would write its new row twice, and duplicate query slots
     // would count the rotation's range errors twice: two launches then)
-    const bool fused = scan || use_step_kernel(k, mode) ||
+    const bool fused = split || scan || use_step_kernel(k, mode) ||
                        (mode != INSITU_TWO_PASS && chunked && !k->vsplit && !k->gpad && chunked_fused_step(g));
     if (fused) {
         StepIn si;
@@ -1093,8 +1133,9 @@ int insitu_cache_debug(insitu_cache *k, int32_t what, int64_t value) {
         if (value == 1 && !k->scan) return fail(INSITU_EINVAL, "the scan attend does not handle this cache");
         if (value == 2 && !k->chunked) return fail(INSITU_EINVAL, "the chunked attend does not handle this cache");
         if (value == 3 && !k->step) return fail(INSITU_EINVAL, "the step kernel does not handle this cache");
-        if (value < 0 || value > 3)
-            return fail(INSITU_EINVAL, "path is 0 (auto), 1 (scan), 2 (chunked) or 3 (step kernel)");
+        if (value == 4 && !k->split) return fail(INSITU_EINVAL, "the split attend does not handle this cache");
+        if (value < 0 || value > 4)
+            return fail(INSITU_EINVAL, "path is 0 (auto), 1 (scan), 2 (chunked), 3 (step kernel) or 4 (split)");
         k->path = (int32_t)value;
         return INSITU_OK;
     case INSITU_DEBUG_PREFILL:

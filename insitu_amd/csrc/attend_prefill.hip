@@ -43,14 +43,13 @@
 // 2,000 243 us (797); 1,000 tokens at d = 128, 3b/3b, two-pass 210 us (1,923), online 265 (1,130).
 #include <type_traits>
 
+#include "digits.h"
 #include "query.h"
 #include "serial_head.h"
 #include "wave.h"
 
 namespace insitu {
 namespace pf {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr double TWO55 = 36028797018963968.0;
 constexpr uint32_t LUT_N = LUT_SPAN + 1;               // p by floor index, the last entry 0
@@ -60,12 +59,6 @@ constexpr float ACC_BOUND = 2147483520.0f;             // the largest float belo
 
 enum Pass { MAXONLY = 0, FIXEDMAX = 1, ONLINE = 2 };
 
-__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
-    return __builtin_amdgcn_perm(hi, lo, sel);         // selector bytes 0-3: lo, 4-7: hi
-}
-__device__ __forceinline__ v4i mma(v4i a, v4i b, v4i c) {
-    return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
-}
 // Bytes b of four words, as the four dwords of bytes 0, 1, 2, 3.
 __device__ __forceinline__ void bytes4(const uint32_t (&z)[4], uint32_t (&o)[4]) {
     const uint32_t a = perm(z[1], z[0], 0x05010400u), b = perm(z[3], z[2], 0x05010400u);
@@ -166,7 +159,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
         for (int i = 0; i < LUT_SPAN / 256; ++i) S.lut[256 * i + tid] = (uint16_t)(x >> i);
         if (tid == 0) S.lut[LUT_SPAN] = 0;
         if (tid < 16) {
-            const uint32_t z = ((uint32_t)kc + 0x808080u) ^ 0x808080u;   // |c| < 2^20
+            const uint32_t z = balanced(kc);   // |c| < 2^20
 #pragma unroll
             for (int l = 0; l < 3; ++l) ((uint8_t *)S.dig[l])[tid] = (uint8_t)(z >> (8 * l));
         }
@@ -206,7 +199,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
                     l1 += ax;
                     rerr += ax >= (uint32_t)Q_ROT_LIMIT ? 1 : 0;
                     big |= ax >> 30;
-                    z[4 * i + j] = ((uint32_t)x[j] + 0x808080u) ^ 0x808080u;
+                    z[4 * i + j] = balanced(x[j]);
                 }
             }
             // byte k of the 16: channel k, or with 4-bit keys the even and the odd channels of 8
@@ -287,42 +280,14 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             const int tok = u % C::ST, b = u / C::ST;
             const int off = b * 16 * kb, wd = off >> 5, sh = off & 31;
             const uint32_t lo = S.raw[bf][tok][wd], hi = S.raw[bf][tok][wd + 1];
-            uint32_t sel[4];
-            if (kb == 4) {
-                sel[0] = lo & 0x0F0F0F0Fu;
-                sel[1] = (lo >> 4) & 0x0F0F0F0Fu;
-                sel[2] = hi & 0x0F0F0F0Fu;
-                sel[3] = (hi >> 4) & 0x0F0F0F0Fu;
-            } else if (kb == 3) {
-                const uint64_t x = (((uint64_t)hi << 32) | lo) >> sh;
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const uint32_t y = (uint32_t)(x >> (12 * w)) & 0xFFFu;
-                    sel[w] = (y & 7u) | (y & 0x38u) << 5 | (y & 0x1C0u) << 10 | (y & 0xE00u) << 15;
-                }
-            } else {
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const uint32_t y = (lo >> (8 * w)) & 0xFFu;
-                    sel[w] = (y & 3u) | (y & 0xCu) << 6 | (y & 0x30u) << 12 | (y & 0xC0u) << 18;
-                }
-            }
+            const uint64_t x = (((uint64_t)hi << 32) | lo) >> sh;
             v4i o[3];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                if (kb == 4) {
-                    const uint32_t top = perm(0u, 0u, ((sel[w] >> 3) & 0x01010101u) + 0x0C0C0C0Cu);   // FF where code >= 8
-                    const uint32_t s7 = sel[w] & 0x07070707u;
-#pragma unroll
-                    for (int l = 0; l < 3; ++l) {
-                        const uint32_t a = perm(dg[l][1], dg[l][0], s7), c = perm(dg[l][3], dg[l][2], s7);
-                        o[l][w] = (int)((a & ~top) | (c & top));
-                    }
-                } else {
-#pragma unroll
-                    for (int l = 0; l < 3; ++l) o[l][w] = (int)perm(dg[l][1], dg[l][0], sel[w]);
-                }
-            }
+            if (kb == 4)
+                expand16<4>(x, dg, o);
+            else if (kb == 3)
+                expand16<3>(x, dg, o);
+            else
+                expand16<2>(x, dg, o);
 #pragma unroll
             for (int l = 0; l < 3; ++l) S.u.op.ka[bf][tok >> 4][l][b >> 2][(b & 3) * 16 + (tok & 15)] = o[l];
         }

@@ -319,6 +319,14 @@ hipError_t launch_step_write(hipStream_t s, const Geom &g, const Tables *t, cons
                              const int32_t *kw, const int32_t *vw, int rounds,
                              const uint64_t (*signs)[2], int32_t *qr, double *qd, int32_t *qok,
                              const int64_t *len_in, int64_t *len_out, DevStats *st);
+// The two-pass attend in two launches (attend_split.hip): one query a sequence, or with step the whole decode step
+// (len the lengths before it); longest: the longest sequence, the new token
+// included.
+bool split_supported(const Geom &g, int64_t capacity);
+size_t split_scratch_bytes(const Geom &g, int64_t capacity);
+hipError_t launch_attend_split(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,
+                               const int64_t *len, ChunkScratch &cs, int64_t longest, const StepIn *step, LaunchEv ev,
+                               DevStats *st);
 // The prefill attend on matrix cores (attend_prefill.hip): query i of n_q (rows of q, (n_q,
 // g.n_q, d)) over rows 0 .. base + i of the sequence at g.base; no scratch, one launch.
 bool prefill_supported(const Geom &g);
