@@ -430,6 +430,9 @@ static Geom chunk_geom(const insitu_cache *k, Geom g) {
     return g;
 }
 
+// The step kernel's: chains of 4 query heads, as the chunked attend sees 8 a KV head.
+static Geom step_geom(const insitu_cache *k, Geom g) { return k->vsplit ? chunk_geom(k, g) : g; }
+
 int insitu_cache_create(insitu_ctx *c, const insitu_cache_desc *desc, insitu_cache **out) {
     if (!c || !desc || !out) return fail(INSITU_EINVAL, "null argument");
     *out = nullptr;
@@ -539,7 +542,6 @@ int insitu_cache_create(insitu_ctx *c, const insitu_cache_desc *desc, insitu_cac
     k->api = desc->chunk_tokens == 512 ? &k_chunk512 : &k_chunk1024;
     k->chunked = k->api->supported(g, desc->capacity);
     k->scan = scan_supported(g, desc->capacity);
-    k->step = step_supported(g, desc->capacity);
     if (!k->chunked && !k->scan && g.G == 8) {
         // 8 query heads a KV head, in a format only the chunked attend takes: as two chains of
         // 4 query heads over the same rows (the rows are read twice, the recurrence is each
@@ -552,12 +554,13 @@ int insitu_cache_create(insitu_ctx *c, const insitu_cache_desc *desc, insitu_cac
         k->chunked = k->api->supported(chunk_geom(k, g), desc->capacity);
         k->gpad = k->chunked;
     }
+    k->step = step_supported(step_geom(k, g), desc->capacity);
     k->split = split_supported(g, desc->capacity);
     if (e == hipSuccess && (k->chunked || k->scan || k->step || k->split)) {
         size_t nb = k->split ? split_scratch_bytes(g, desc->capacity) : 0;
         if (k->step) {
             k->step_mc = step_max_chunks(desc->capacity);
-            const size_t nk = step_scratch_bytes(g, k->step_mc);
+            const size_t nk = step_scratch_bytes(step_geom(k, g), k->step_mc);
             nb = nk > nb ? nk : nb;
         }
         if (k->chunked) {
@@ -709,8 +712,10 @@ static bool use_scan(const insitu_cache *k, int32_t mode) {
 }
 
 // The fused decode step's own kernel (attend_step.hip), sequential and split mode, wherever
-// it handles the format (d = 64, 4 query heads per KV head, 4-bit keys, 2-bit values, up to
-// 512 chunks of 1,024 tokens); the test hook can pin the chunked (2) or scan (1) attend.
+// it handles the format (d = 64, 4 or 3-bit keys, 2-bit values, 4 query heads per KV head, or 8
+// where the chunked attend sees them as two chains; up to 512 chunks of 1,024 tokens); the test
+// hook can pin the chunked (2) or scan (1) attend. No slower anywhere from 30 to 32,768 tokens and
+// 1 to 64 sequences in the four formats (the kernel's figures).
 static bool use_step_kernel(const insitu_cache *k, int32_t mode) {
     if ((mode != INSITU_SEQUENTIAL && mode != INSITU_SPLIT) || !k->step) return false;
     return k->path != 1 && k->path != 2;
@@ -782,7 +787,7 @@ static int attend_impl(insitu_cache *k, const int32_t *q, int32_t *out, int32_t 
         k->scr.spin_limit = k->spin_limit;
         int64_t longest = 0;
         for (int64_t n : k->len_host) longest = n > longest ? n : longest;
-        HIP_TRY(launch_step(k->ctx->stream, k->g, k->tabs, out, len, k->scr, ep, k->step_mc,
+        HIP_TRY(launch_step(k->ctx->stream, step_geom(k, k->g), k->tabs, out, len, k->scr, ep, k->step_mc,
                             step_max_chunks(longest + 1), *step, ev, k->stats),
                 "step launch");
         return INSITU_OK;

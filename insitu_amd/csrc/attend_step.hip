@@ -1,7 +1,14 @@
 // The fused decode step (kernel.py:271-345): rotate q/k/v, encode and append the
 // token's k/v row, then attend_online (ops/attention.py:451-513) and the finalize
 // (:873-880) over every cached row, bit-exact, in one launch of 16-wave workgroups,
-// one per (1,024-token chunk, sequence, KV head) at d = 64, 4 query heads per KV head.
+// one per (1,024-token chunk, sequence, chain) at d = 64; a chain is a KV head's 4 query heads, or
+// 4 of its 8. 4-bit keys; 3-bit ones are widened in registers (some 70 instructions a token against
+// the score's 300), so that the score stays one path: an LDS read for the centroids of two channels.
+// Bounds: the chain of dependent phases up to some 8,192 tokens, then the fp64 scores and the walk.
+// Steps with 3-bit keys, 2,047 tokens, before (the chunked attend: with 8 query heads a write launch
+// and an attend launch, 2 chains a KV head either way) and here, flat and peaked weights: 4 heads
+// 35 -> 33 and 22 -> 21 us, x 64 sequences 203 -> 147 and 156 -> 96; 8 heads (4 KV heads) 47 -> 33 and
+// 28 -> 21, x 64 sequences 179 -> 147 and 103 -> 96.
 //
 // The arithmetic is the chunked attend's (attend_chunked.hip): a chunk knows the
 // running maximum before it (M_in, by a decoupled look-back over its predecessors'
@@ -277,13 +284,13 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
                                                      StepIn si) {
     using L = StepLds<KB, VB>;
     constexpr int NV = 1 << VB, NK = 1 << KB;
-    constexpr int KWORDS = D * KB / 32, VWORDS = D * VB / 32;
+    // a row's key codes in registers: 4 bits each, whatever the cache's width (see widen)
+    constexpr int KWORDS = D * 4 / 32, VWORDS = D * VB / 32;
     constexpr int KBYTES = D * KB / 8;
     constexpr int NFULL = KBYTES / 16, HALF = (KBYTES % 16) / 8;
     constexpr int KPL = NFULL + HALF;         // key planes; the value plane follows, then the norms
     static_assert(VB == 1 || VB == 2, "one value plane of 8 or 16 bytes");
-    static_assert(KB == 4, "the score's channel slices take 8 codes a word, 2 planes a row");
-    static_assert(32 % KB == 0 && 32 % VB == 0, "the new row's codes never straddle a word");
+    static_assert((KB == 4 || KB == 3) && 32 % VB == 0, "the key widths widen and the new row's packing know");
     static_assert(KWORDS <= D * 4 / 32 && VWORDS <= D * 2 / 32, "new-row staging sizes");
     __shared__ L S;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -322,6 +329,9 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     // entries in LDS; it still takes every barrier and its share of the walk.
     const bool wlive = t0 + 64 * wv < T;
     if (own && kvh == 0 && tid == 0) si.len_out[b] = T;
+    // a KV head seen as several chains: every one encodes the new row and stores the same words, the
+    // first one counts its range errors
+    const bool row_owner = (kvh & ((1 << g.kv_shift) - 1)) == 0;
     const int score_shift = CENT_FRAC + g.norm_frac;
     const uint8_t *hb = plane_ptr(g, b, kvh, 0);
 
@@ -333,7 +343,8 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     // paths join, before their planes go out), the score's table, the planes. A wait for a
     // later load waits for every earlier one.
     const int32_t *xsrc = wv < G ? si.qw + ((int64_t)b * g.n_q + kvh * G + wv) * D
-                                 : (wv == G + 1 ? si.vw : si.kw) + ((int64_t)b * g.n_kv + kvh) * D;
+                                 : (wv == G + 1 ? si.vw : si.kw) +
+                                       ((int64_t)b * (g.n_kv >> g.kv_shift) + (kvh >> g.kv_shift)) * D;
     const int32_t xv = xsrc[lane];
     // the new token's encoder: lane i < 2^bits - 1 of wave G (keys) and G + 1 (values) holds
     // boundary i (quantize.py:183-196)
@@ -444,7 +455,7 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
         const int f = wv - G;      // 0: key, 1: value
         int32_t r[1];
         const int32_t in[1] = {xv};
-        rotate_loaded<1>(in, D, si.rounds, si.sg, r, &st->range_errors);
+        rotate_loaded<1>(in, D, si.rounds, si.sg, r, row_owner ? &st->range_errors : nullptr);
         const int64_t x[1] = {r[0]};
         const int64_t n = norm_wire<1>(x, D, g.norm_frac);
         // code = #{i : (x << 8) > norm * b_i}, the products norm * b_i broadcast from their lanes
@@ -458,7 +469,7 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
         // Pack: a word holds 32 / bits consecutive codes, LSB first (quantize.py:271-289): each
         // lane shifts its code into place, an OR over its group of lanes (lane xor 1, 2, ...)
         // gives the word in every lane of the group, and the group's first lane stores it.
-        const int bits = f == 0 ? KB : VB;
+        const int bits = f == 0 ? 4 : VB;
         const int per = 32 / bits;                                  // codes per word
         uint32_t wword = (uint32_t)code << (bits * (lane & (per - 1)));
         wword |= xor_lane32<1>(wword, lane);
@@ -470,7 +481,9 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
         uint8_t *const rowb = plane_ptr(g, b, kvh, 0);            // writable
         uint16_t *nword = (uint16_t *)(rowb + (KPL + 1) * g.span + (T - 1) * 4);
         if ((lane & (per - 1)) == 0) {
-            if (f == 0) {
+            if (f == 0 && KB == 3) {
+                S.nk[wi] = wword;
+            } else if (f == 0) {
                 // key word wi: plane wi / 4, word wi % 4 of the token's 16 bytes (8 in a half plane)
                 const int pw = wi / 4 < NFULL ? 16 : 8;
                 pub32(rowb + (wi / 4) * g.span + (T - 1) * pw + 4 * (wi % 4), wword);
@@ -479,6 +492,19 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
                 pub32(rowb + KPL * g.span + (T - 1) * (VWORDS * 4) + 4 * wi, wword);
                 S.nv[wi] = wword;
             }
+        }
+        if (KB == 3 && f == 0) {
+            // 3-bit codes: 24 bits from each group of 8 lanes; lane wi puts word wi together from the
+            // two groups its 32 bits lie in
+            uint32_t grp8 = (uint32_t)code << (3 * (lane & 7));
+            grp8 |= xor_lane32<1>(grp8, lane);
+            grp8 |= xor_lane32<2>(grp8, lane);
+            grp8 |= xor_lane32<4>(grp8, lane);
+            const int i0 = 32 * lane / 24, off = 32 * lane - 24 * i0;
+            const uint32_t lo = (uint32_t)__shfl((int)grp8, 8 * i0), hi = (uint32_t)__shfl((int)grp8, 8 * i0 + 8);
+            const int pw = lane < 4 * NFULL ? 16 : 8;
+            if (lane < KBYTES / 4)
+                pub32(rowb + (lane / 4) * g.span + (T - 1) * pw + 4 * (lane % 4), lo >> off | hi << (24 - off));
         }
         if (lane == 0) {
             __hip_atomic_store(nword + f, (uint16_t)(n & 0xFFFF), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -495,6 +521,21 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     int32_t ex = 0;
     if (tid >= 320 && tid < 320 + NV) tab = tabs->vc[tid - 320];
     if (tid >= 384 && tid < 384 + 256) ex = tabs->exp_table[tid - 384];
+    if constexpr (KB == 3) {
+        // 8 codes of 3 bits to 8 of 4: the score then takes one path (two centroids an LDS read by
+        // code byte), for some 9 instructions a word
+        uint32_t raw[KBYTES / 4 + 1];
+#pragma unroll
+        for (int i = 0; i <= KBYTES / 4; ++i) raw[i] = i < KBYTES / 4 ? kw[i] : 0u;
+#pragma unroll
+        for (int i = 0; i < KWORDS; ++i) {
+            const int w = 24 * i / 32;
+            uint32_t y = __builtin_amdgcn_alignbit(raw[w + 1], raw[w], 24 * i % 32);
+            y = (y & 0xFFFu) | (y & 0xFFF000u) << 4;
+            y = (y & 0x003F003Fu) | (y & 0x0FC00FC0u) << 2;
+            kw[i] = (y & 0x07070707u) | (y & 0x38383838u) << 1;
+        }
+    }
     if (slice > 0) {
         // a helper's slice of its token's key words: word w0 on (uniform selects over the row)
         const int w0 = cps >= 8 ? slice * cps / 8 : slice / 2;
@@ -545,7 +586,6 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     auto score_steps = [&](auto ns) __attribute__((always_inline)) {
         constexpr int NS = decltype(ns)::value;
         constexpr int NQ = NS / 2;                                  // query registers
-        static_assert(KB == 4, "the score reads two 4-bit codes' centroids by code byte");
         double(&ac)[G] = acc;
         int32_t qi[NQ];
         {
@@ -1693,7 +1733,7 @@ bool step_supported(const Geom &g, int64_t capacity) {
     using namespace stepk;
     const int kbytes = g.d * g.kb / 8;
     const int kpl = kbytes / 16 + (kbytes % 16) / 8;
-    return g.d == D && g.G == G && g.kb == 4 && g.vb == 2 && g.n_planes == kpl + 2 &&
+    return g.d == D && g.G == G && (g.kb == 4 || g.kb == 3) && g.vb == 2 && g.gq == 0 && g.n_planes == kpl + 2 &&
            (capacity + CHUNK - 1) / CHUNK <= HMAX && g.norm_frac == 9;
 }
 
@@ -1760,6 +1800,9 @@ hipError_t launch_step(hipStream_t s, const Geom &g, const Tables *t, int32_t *o
     dim3 grid((unsigned)(grid_chunks * chains)), block(NT);
     if (g.kb == 4 && g.vb == 2)
         hipExtLaunchKernelGGL((step_kernel<4, 2>), grid, block, 0, s, ev.start, ev.stop, 0, g, t, out, len, ck, st,
+                              si);
+    else if (g.kb == 3 && g.vb == 2)
+        hipExtLaunchKernelGGL((step_kernel<3, 2>), grid, block, 0, s, ev.start, ev.stop, 0, g, t, out, len, ck, st,
                               si);
     else
         return hipErrorInvalidValue;
