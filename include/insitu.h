@@ -298,9 +298,11 @@ enum {
                                         4 two-pass mode's split attend
                                         (any other mode automatic);
                                         INSITU_EINVAL if the kernel does not handle the cache   */
-    INSITU_DEBUG_APPEND = 5,         /* the append's kernel: 0 automatic (lane = row where it
-                                        handles the format: d = 64, 4/2- or 2/2-bit codes), 1 the
-                                        lane-per-channel kernel for every format                */
+    INSITU_DEBUG_APPEND = 5,         /* the append's kernel: 0 automatic (lane = row for more
+                                        than 4,096 rows where it handles the format: d = 64, 4/2-
+                                        or 2/2-bit codes), 1 the lane-per-channel kernel for every
+                                        format, 2 lane = row however few the rows, where it
+                                        handles the format                                      */
     INSITU_DEBUG_PREFILL = 6         /* the causal attends' kernel: 0 automatic (the prefill kernel
                                         where it handles the format and the queries fill it), 1 the
                                         decode attends over a virtual batch, 2 the prefill kernel;

@@ -193,7 +193,7 @@ struct insitu_cache {
     int32_t spin_limit = 1 << 20;         // insitu_cache_debug
     int32_t path = 0;                     // insitu_cache_debug: 0 auto, 1 scan, 2 chunked, 3 step kernel, 4 split
     int32_t prefill_path = 0;             // insitu_cache_debug: 0 auto, 1 virtual batch, 2 prefill kernel
-    int32_t append_path = 0;              // insitu_cache_debug: 0 auto, 1 the lane-per-channel kernel
+    int32_t append_path = 0;              // insitu_cache_debug: 0 auto, 1 the lane-per-channel kernel, 2 lane = row
 };
 
 namespace {
@@ -671,7 +671,7 @@ static int append_impl(insitu_cache *k, int seq_lo, int seq_hi, const int32_t *k
     HIP_TRY(launch_append(k->ctx->stream, k->g, k->tabs, kr, vr, n_tok, seq_lo, seq_hi,
                           k->len_dev[k->cur], k->len_dev[k->cur ^ 1], k->stats,
                           wire ? k->desc.fmt.rot_rounds : 0, wire ? k->desc.fmt.rot_signs : nullptr,
-                          k->append_path == 0 ? &k->tabs_host : nullptr),
+                          k->tabs_host, k->append_path),
             "append launch");
     k->cur ^= 1;
     for (int b = seq_lo; b < seq_hi; ++b) k->len_host[b] += n_tok;
@@ -1149,7 +1149,8 @@ int insitu_cache_debug(insitu_cache *k, int32_t what, int64_t value) {
         k->prefill_path = (int32_t)value;
         return INSITU_OK;
     case INSITU_DEBUG_APPEND:
-        if (value < 0 || value > 1) return fail(INSITU_EINVAL, "append kernel is 0 (auto) or 1 (lane per channel)");
+        if (value < 0 || value > 2)
+            return fail(INSITU_EINVAL, "append kernel is 0 (auto), 1 (lane per channel) or 2 (lane = row)");
         k->append_path = (int32_t)value;
         return INSITU_OK;
     default:

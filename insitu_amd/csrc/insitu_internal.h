@@ -199,11 +199,12 @@ hipError_t launch_exp_lut(hipStream_t s, const Tables *t, const int64_t *delta, 
 hipError_t launch_finalize(hipStream_t s, const int64_t *acc, const int64_t *l, int rows, int d,
                            int64_t *out, int64_t *recip, int32_t *shift);
 // Append n_tok rows of k/v ([seq][tok][kv head][d], int32) to sequences [seq_lo, seq_hi);
-// rounds > 0 rotates them first (wire rows, rotate.py:170-197, `signs` as launch_rotate's).
+// rounds > 0 rotates them first (wire rows, rotate.py:170-197, `signs` as launch_rotate's); path:
+// the kernel, 0 automatic, 1 the lane-per-channel one, 2 lane = row where it handles the format.
 hipError_t launch_append(hipStream_t s, const Geom &g, const Tables *t, const int32_t *k,
                          const int32_t *v, int n_tok, int seq_lo, int seq_hi, const int64_t *len_in,
-                         int64_t *len_out, DevStats *st, int rounds = 0,
-                         const uint64_t (*signs)[2] = nullptr, const Tables *host_tabs = nullptr);
+                         int64_t *len_out, DevStats *st, int rounds, const uint64_t (*signs)[2],
+                         const Tables &host_tabs, int path);
 bool chunked_supported(const Geom &g, int64_t capacity);
 int64_t chunked_max_chunks(int64_t capacity);
 int64_t chunked_pool_slots(int64_t max_chunks);

@@ -687,7 +687,12 @@ hipError_t launch_step_write(hipStream_t s, const Geom &g, const Tables *t, cons
 // bits (instantiated here for 4/2 and 2/2); the boundaries non-decreasing (4-bit codes are
 // found by bisection); every boundary below 2^24 in magnitude and the
 // encoder's shift CENT_FRAC + norm_frac - QK_FRAC at least 0 (its int32 thresholds are then
-// exact); k and v 16-byte aligned (whole-wave 16-byte loads); fewer than 2^31 rows.
+// exact); k and v 16-byte aligned (whole-wave 16-byte loads); fewer than 2^31 rows. It takes 64 rows a
+// wave: automatically only where that leaves no SIMD idle that a row a wave would use. A few rows
+// take it 17.9 us (4/2-bit codes) or 15.3 us (2/2) whatever their number, a lone wave's 5,000
+// instructions; a row a wave 11.9 us up to 2,664 rows. At 4,096 rows 14.3 against 18.1 us (4/2, 8 KV
+// heads) and 13.6 against 15.5 (2/2); at 8,192 21.2 against 17.6 and 20.0 against 15.3.
+constexpr int64_t AR_MIN_ROWS = 4096;
 bool append_rows_ok(const Geom &g, const Tables &th, const int32_t *k, const int32_t *v, int64_t rows) {
     if (g.d != 64 || rows >= (int64_t(1) << 31) - 64) return false;
     if (!((g.kb == 4 && g.vb == 2) || (g.kb == 2 && g.vb == 2))) return false;
@@ -705,12 +710,12 @@ bool append_rows_ok(const Geom &g, const Tables &th, const int32_t *k, const int
 hipError_t launch_append(hipStream_t s, const Geom &g, const Tables *t, const int32_t *k,
                          const int32_t *v, int n_tok, int seq_lo, int seq_hi, const int64_t *len_in,
                          int64_t *len_out, DevStats *st, int rounds, const uint64_t (*signs)[2],
-                         const Tables *host_tabs) {
+                         const Tables &host_tabs, int path) {
     const int64_t rows = (int64_t)(seq_hi - seq_lo) * n_tok * g.n_kv;
     if (rows <= 0) return hipSuccess;
     if (rounds < 0 || rounds > 2 || (rounds && !signs)) return hipErrorInvalidValue;
     const RotSigns sg = rounds ? rot_signs(rounds, signs) : RotSigns{};
-    if (host_tabs && append_rows_ok(g, *host_tabs, k, v, rows)) {
+    if (path != 1 && (path == 2 || rows > AR_MIN_ROWS) && append_rows_ok(g, host_tabs, k, v, rows)) {
         const int waves = (int)((rows + 63) / 64);
         dim3 grid((unsigned)((waves + AR_WAVES - 1) / AR_WAVES)), block(64 * AR_WAVES);
         const int nr = (int)rows;
@@ -725,8 +730,10 @@ hipError_t launch_append(hipStream_t s, const Geom &g, const Tables *t, const in
 #undef INSITU_AR
         return hipGetLastError();
     }
-    // about 8 rows a wave at the most, 4 waves a workgroup, up to 8 workgroups a CU
-    int64_t blocks = (rows + 8 * APPEND_WAVES - 1) / (8 * APPEND_WAVES);
+    // A row a wave as long as that fills no more than 8 workgroups a CU, 4 waves a workgroup: 64 tokens
+    // of 8 KV heads take 12.2 us in 4/3-bit codes at d = 64 and 14.7 us in 3/3-bit codes at d = 128 (42.9
+    // and 49.9 at 8 rows a wave); 4,096 tokens 54.2 and 72.1 us (58.9 and 77.2).
+    int64_t blocks = (rows + APPEND_WAVES - 1) / APPEND_WAVES;
     if (blocks > 2048) blocks = 2048;
     if (blocks < 1) blocks = 1;
     dim3 grid((unsigned)blocks), block(64 * APPEND_WAVES);
