@@ -42,11 +42,13 @@
 // walks them from chunk 0's state, finalizes and writes Q16. Chunk 0 counts
 // itself done before publishing its state, so when it is the last (it usually
 // is: it holds most rescale events) the state never leaves its registers.
-// Scores: sum_ch q[ch] * c[code_ch] in fp64 FMA -- every partial sum is an
-// integer below 2^51, so it is exact -- then the int64 norm multiply and >>24
-// of the reference.
+// Scores: sum_ch q[ch] * c[code_ch] exactly, on the matrix cores as sums of 8-bit
+// digits' products, or (the fused step and the two-pass maxima) in fp64 FMA, whose
+// partial sums are integers below 2^51; then the int64 norm multiply and >>24 of
+// the reference.
 #include <type_traits>
 
+#include "digits.h"
 #include "query.h"
 #include "row_codec.h"
 #include "serial_head.h"
@@ -225,17 +227,21 @@ struct ChunkLds {
     struct Replay {
         uint16_t slot[GF][NSEG];   // the runs in order: slot | RUN_EVENT when a rescale opens it
     };
-    union {
+    union alignas(16) {            // 16-byte aligned: the score stages rows as 128-bit words
         Phase ph;
         Replay rp;
         SerialLds<KF<D, KB>::RS> fb[GF];
     } u;
     typename std::conditional<STEP, StepLds<D>, NoStep>::type nr;
     union alignas(16) {            // 16-byte aligned: the score loop reads the rows as 128-bit words
-        double qf[D * GF];         // the group's query rows [c][h] (unless staged), until the scores
+        struct {
+            double qf[D * GF];     // the group's query rows [c][h] (unless staged), until the scores
+            int32_t qb[GF * D];    // the same [h][c] as balanced digits, except in the fused step
+        } s;
         int32_t tt[GF][64][8];     // run sums: a block of 64 entries' terms for every value code
     } qt;
     double kcf[16];
+    alignas(16) uint32_t dig[3][4];    // the key centroids' balanced digits (digits.h)
     int64_t kc[16];
     int64_t vc[16];
     int32_t vc32[16];
@@ -359,6 +365,118 @@ __device__ __forceinline__ void score_keys(const uint32_t (&w)[TPT][KF<D, KB>::K
     }
 }
 
+// The same scores on the matrix cores, except in the fused step: a head's four balanced digits are
+// four rows, so the GF heads fill the 16 rows, against the centroid digits of 16 tokens (digits.h).
+// The digit sums make the int64 dot exactly, whatever the rows. A wave scores its own tokens, half
+// of them at a time: their lanes' key words go to LDS (kbuf, the wave's share of the value rows,
+// which are staged after the scores), from where lane (token, quarter of the channels) takes its
+// codes, and the dots come back through dbuf (the wave's share of the candidate records) to the
+// lanes that own the tokens. A centroid then costs a byte permute for each of its 3 digits and 4
+// channels, where the fp64 score reads 8 bytes of LDS and issues 4 FMAs a (token, channel): a CU's LDS
+// and its FMAs bounded the attend of large batches. 16 sequences of 131,072 rows, d = 128, 3-bit keys
+// and values: 739 us a call (810 with the fp64 score; 2.3 TB/s); 64 of 1,024 to 8,192 rows, d = 64,
+// 4/2 bits: 111.3 (112.5: its chunks are few a CU, and the chain of phases behind the score bounds it).
+template <int D, int KB>
+__device__ __forceinline__ void score_mfma(const uint32_t (&w)[TPT][KF<D, KB>::KWORDS + 1],
+                                           const uint32_t (&normw)[TPT], const int32_t *qb,
+                                           const uint32_t (*dig)[4], uint32_t *kbuf, int64_t *dbuf,
+                                           int score_shift, int64_t (&s)[TPT][GF]) {
+    constexpr int KW = KF<D, KB>::KWORDS, NT = 32 * TPT, CPL = D / 64;
+    static_assert(KW % 2 == 0, "rows are stored as 8 or 16 bytes");
+    static_assert(NT * KW <= 2 * NT * KF<D, KB>::VW, "half the wave's key rows fit its value rows");
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4, own = lane & 31;
+    // the query operand: lane = (head, digit), the channels of a quarter
+    v4i qa[CPL];
+    const uint32_t dgt = lane & 3, s01 = 0x0C0C0000u | dgt | (4u + dgt) << 8, s23 = 0x00000C0Cu | dgt << 16 | (4u + dgt) << 24;
+#pragma unroll
+    for (int b = 0; b < CPL; ++b) {
+        int32_t x[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int4 v = *(const int4 *)(qb + (col >> 2) * D + grp * (D / 4) + 16 * b + 4 * i);
+            x[4 * i] = v.x;
+            x[4 * i + 1] = v.y;
+            x[4 * i + 2] = v.z;
+            x[4 * i + 3] = v.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            qa[b][i] = (int)(perm((uint32_t)x[channel_of(KB, 4 * i + 1)], (uint32_t)x[channel_of(KB, 4 * i)], s01) |
+                             perm((uint32_t)x[channel_of(KB, 4 * i + 3)], (uint32_t)x[channel_of(KB, 4 * i + 2)], s23));
+    }
+    uint32_t dg[3][4];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dg[i][j] = dig[i][j];
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+        const bool mine = lane >> 5 == half;
+        wave_sync();
+        if (mine) {
+#pragma unroll
+            for (int j = 0; j < TPT; ++j) {
+                uint32_t *to = kbuf + (own * TPT + j) * KW;
+                if constexpr (KW % 4 == 0) {
+#pragma unroll
+                    for (int i = 0; i < KW; i += 4) *(uint4 *)(to + i) = make_uint4(w[j][i], w[j][i + 1], w[j][i + 2], w[j][i + 3]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < KW; i += 2) *(uint2 *)(to + i) = make_uint2(w[j][i], w[j][i + 1]);
+                }
+            }
+        }
+        wave_sync();
+#pragma unroll 2
+        for (int tile = 0; tile < NT / 16; ++tile) {       // (by 4 it takes 3 to 10 registers more than there are)
+            // channels [grp D / 4, (grp + 1) D / 4) of token `col` of the tile
+            const uint32_t *row = kbuf + (16 * tile + col) * KW;
+            uint64_t code[CPL];
+            if constexpr (KB == 4) {
+#pragma unroll
+                for (int b = 0; b < CPL; ++b)
+                    code[b] = (uint64_t)row[(grp * CPL + b) * 2] | (uint64_t)row[(grp * CPL + b) * 2 + 1] << 32;
+            } else if constexpr (KB == 3 && D == 64) {
+                const int i = (3 * grp) >> 1;
+                code[0] = ((uint64_t)row[i] | (uint64_t)row[i + 1] << 32) >> (16 * (grp & 1));
+            } else if constexpr (KB == 3) {
+                const uint32_t a = row[3 * grp], c = row[3 * grp + 1], e = row[3 * grp + 2];
+                code[0] = (uint64_t)a | (uint64_t)c << 32;
+                code[1] = ((uint64_t)c | (uint64_t)e << 32) >> 16;
+            } else {
+#pragma unroll
+                for (int b = 0; b < CPL; ++b) code[b] = row[grp * CPL + b];
+            }
+            v4i T[3];
+#pragma unroll
+            for (int l = 0; l < 3; ++l) T[l] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int b = 0; b < CPL; ++b) {
+                v4i o[3];
+                expand16<KB>(code[b], dg, o);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) T[l] = mma(qa[b], o[l], T[l]);
+            }
+            // lane = (token, head), registers the row's digits. Centroids are below 2^20, so that
+            // every 32-bit sum here stays below 2^31.
+            const int32_t lo = T[0][0] + ((T[0][1] + T[1][0]) << 8);
+            const int32_t mid = T[0][2] + T[1][1] + T[2][0] + ((T[0][3] + T[1][2] + T[2][1]) << 8);
+            const int32_t top = T[1][3] + T[2][2] + (T[2][3] << 8);
+            // (the odd heads' 16 tokens apart by 16, so that their stores miss the even heads' banks)
+            dbuf[grp * NT + ((16 * tile + col) ^ (16 * (grp & 1)))] = (int64_t)mid * 65536 + lo + ((int64_t)top * (1ll << 32));
+        }
+        wave_sync();
+        if (mine) {
+#pragma unroll
+            for (int h = 0; h < GF; ++h)
+#pragma unroll
+                for (int j = 0; j < TPT; ++j)
+                    s[j][h] = wmul(dbuf[h * NT + ((own * TPT + j) ^ (16 * (h & 1)))], sext16(normw[j])) >> score_shift;
+        }
+    }
+    wave_sync();
+}
+
 // ---------------------------------------------------------------------------
 // two-pass pre-pass: the maximum score of every chunk, and the score statistics
 // ---------------------------------------------------------------------------
@@ -475,7 +593,7 @@ __global__ void __launch_bounds__(CT) chunk_max_kernel(Geom g, const Tables *__r
 // the workgroup of the chunk holding the new token rotates, encodes and packs
 // its key/value row, stores it into the planes and scores it from LDS.
 template <int D, int KB, bool SEQ, bool QS, bool STEP>
-__global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__restrict__ tabs,
+__global__ void __launch_bounds__(CT, SEQ && D > 64 ? 4 : 2) chunk_kernel(Geom g, const Tables *__restrict__ tabs,
                                                    const int32_t *__restrict__ q,
                                                    const double *__restrict__ qd,
                                                    const int32_t *__restrict__ qok, int32_t *out,
@@ -522,6 +640,11 @@ __global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__re
         const int64_t vc_t = tid < nv ? tabs->vc[tid] : 0;
         const int32_t ex_t = tid < 256 ? tabs->exp_table[tid] : 0;
         int32_t q_t[D / 64];
+        double qd_t = 0.0;
+        if constexpr (QS) {
+            static_assert(GF * D <= CT, "a staged query value a thread");
+            if (tid < GF * D) qd_t = qd[(int64_t)chain * D * GF + tid];
+        }
         int32_t kv_t[D / 64];          // STEP: the new token's key (wave GF) or value (GF + 1)
         if (STEP) {
             if (wv < GF)
@@ -557,10 +680,17 @@ __global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__re
         if (tid < 16) {
             S.kc[tid] = kc_t;
             S.kcf[tid] = (double)kc_t;
+            if constexpr (!STEP) {
+                const uint32_t z = balanced((int32_t)kc_t);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) ((uint8_t *)S.dig[l])[tid] = (uint8_t)(z >> (8 * l));
+            }
             S.vc[tid] = vc_t;
             S.vc32[tid] = (int32_t)vc_t;               // |centroid| < 2^18 (Q1.15)
         }
         if (tid < 256) S.expt[tid] = ex_t;
+        if constexpr (QS)
+            if (tid < GF * D) S.qt.s.qb[(tid % GF) * D + tid / GF] = (int32_t)balanced((int32_t)qd_t);
         if (wv == 0) {
             const int64_t m = wave_max_i64(vc_t < 0 ? -vc_t : vc_t);
             if (lane == 0) S.vcmax = m;
@@ -590,25 +720,26 @@ __global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__re
         }
         __syncthreads();
         // Whether every score of the group stays an exact fp64 integer (query.h).
-        const double *qc = qd + (int64_t)chain * D * GF;
         bool ok;
         if constexpr (QS) {
             ok = qok[chain] != 0;
         } else {
             // Chunk 0 counts the range errors of the rotated queries, once per call.
             if (wv < GF) {
-                const bool okh = stage_query_head<D / 64>(q_t, D, wv, S.qt.qf, tabs->kc_absmax,
+                const bool okh = stage_query_head<D / 64>(q_t, D, wv, S.qt.s.qf, tabs->kc_absmax,
                                                           chunk == 0 && real_head(g, wv) ? &st->range_errors
                                                                                          : nullptr);
                 if (lane == 0 && !okh) atomicAnd(&S.qok, 0);
                 if constexpr (STEP) {
 #pragma unroll
                     for (int k = 0; k < D / 64; ++k) S.nr.qi[wv][lane + 64 * k] = q_t[k];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < D / 64; ++k) S.qt.s.qb[wv * D + lane + 64 * k] = (int32_t)balanced(q_t[k]);
                 }
             }
             __syncthreads();
             ok = S.qok != 0;
-            qc = S.qt.qf;
         }
         // The fused step's new token, beside the score phase: wave 0 encodes its
         // key (rotated by wave GF), stores the key words into the planes and
@@ -648,7 +779,7 @@ __global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__re
 #pragma unroll
                             for (int k = 0; k < D / 64; ++k) {
                                 const int c = lane + 64 * k;
-                                a = fma(S.qt.qf[c * GF + h], S.kcf[S.nr.codes[0][c]], a);
+                                a = fma(S.qt.s.qf[c * GF + h], S.kcf[S.nr.codes[0][c]], a);
                             }
                             part[h] = dbl_to_i64(a);
                         }
@@ -691,7 +822,11 @@ __global__ void __launch_bounds__(CT, 2) chunk_kernel(Geom g, const Tables *__re
         for (int h = 0; h < GF; ++h) mx[h] = nmx[h];
         if (ok) {
             int64_t s[TPT][GF];
-            score_keys<D, KB>(kw, nw, qc, S.kcf, score_shift, s);
+            if constexpr (STEP)
+                score_keys<D, KB>(kw, nw, S.qt.s.qf, S.kcf, score_shift, s);
+            else
+                score_mfma<D, KB>(kw, nw, S.qt.s.qb, S.dig, (uint32_t *)S.u.ph.vw[64 * TPT * wv],
+                                  (int64_t *)(&S.u.ph.rec[0][0] + 64 * TPT * GF * wv), score_shift, s);
             unsigned long long ovf = novf;
             int64_t mabs = nmabs;
 #pragma unroll

@@ -23,13 +23,15 @@ constexpr double DOT_LIMIT = 2251799813685248.0;     // 2^51
 // c's rotated value. Writes the head's fp64 column of the block qdc (global
 // staging or a workgroup's LDS copy), counts values beyond the +-2^27 the
 // 24-bit seam can produce as range errors (unless range_err is null), and
-// returns (wave-uniform) whether the head's scores stay exact.
+// returns (wave-uniform) whether the head's scores stay exact: also not where a value has no
+// balanced digits (digits.h), 32 times and more beyond that range.
 template <int CPL>
 __device__ __forceinline__ bool stage_query_head(const int32_t (&v)[CPL], int d, int h,
                                                  double *qdc, double kc_absmax,
                                                  unsigned long long *range_err) {
     const int lane = threadIdx.x & 63;
     int64_t l1 = 0, bad = 0;
+    bool wide = false;
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
         const int c = lane + 64 * k;
@@ -38,12 +40,13 @@ __device__ __forceinline__ bool stage_query_head(const int32_t (&v)[CPL], int d,
             qdc[c * GF + h] = (double)x;
             l1 += x < 0 ? -x : x;
             bad += (x >= Q_ROT_LIMIT || x <= -Q_ROT_LIMIT) ? 1 : 0;
+            wide = wide || x > 0x7FFFFFFFll - 0x808080;
         }
     }
     l1 = wave_sum_i64(l1);          // < 2^38: exact as a double below
     bad = wave_sum_i64(bad);
     if (range_err && lane == 0 && bad) atomicAdd(range_err, (unsigned long long)bad);
-    return (double)l1 * kc_absmax < DOT_LIMIT;
+    return (double)l1 * kc_absmax < DOT_LIMIT && __ballot(wide) == 0;
 }
 
 }  // namespace insitu
