@@ -870,19 +870,34 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 // Whether a causal attend runs on the prefill kernel (attend_prefill.hip). Its waves walk their
 // rows' whole contexts, so a grid that does not fill the chip takes a time of its own in the
 // context's length alone; the chunked attend over a virtual batch spreads one query's context over
-// the chip and takes time in proportion to the queries. Fitted to both, measured over 1 to 256
-// queries and 128 to 32,768 rows (us, 32 query heads; e.g. 16 queries of 2,048 rows at d = 64:
-// 214 here, 68 there; 128: 218 and 275; 256 of 32,768: 2,514 and 7,106).
+// the chip and takes time in proportion to the queries, once they are enough to show over its chain
+// of phases. Fitted to both, measured over 1 to 512 queries of 16 to 4,096 rows, 32 query heads, in
+// 4/2- and 3/2-bit codes at d = 64 and 3/3 and 4/2 at d = 128, online and two-pass: the choice takes
+// 0.5 % longer than the better kernel in the mean of them, 1.3 times as long at the worst. E.g. here /
+// there us, d = 64, online: 16 queries of 64 rows 25/27, 256 rows 50/35, 2,048 rows 220/68; 128 of
+// 256 rows 50/83, of 2,048 rows 221/273; d = 128, 3/3 bits: 64 of 512 rows 157/96, 192 263/408 of 1,024.
 static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
     if (mode == INSITU_SERIAL || !prefill_supported(gv) || k->prefill_path == 1) return false;
     if (k->prefill_path == 2) return true;
     if (k->path != 0 && k->path != 4) return false;
     if (!k->chunked) return true;           // else token by token
     const bool two = mode == INSITU_TWO_PASS, d64 = gv.d == 64;
-    const double t = (double)(base + n_q);
-    const double here = (two ? 14.0 : 20.0) + t * (d64 ? 0.075 : 0.16) * (two ? 1.2 : 1.0);
-    const double there = (d64 ? 28.0 : 40.0) + 25.0 * (t < 1500.0 ? t / 1500.0 : 1.0) +
-                         t * (double)n_q * gv.n_q * (d64 ? 2.65e-5 : 5.2e-5) * (two ? 1.95 : 1.0);
+    const double t = (double)(base + n_q), near = t < 1024.0 ? t : 1024.0, n = (double)n_q;
+    // (3-bit codes at d = 128 take most to load and widen; few waves walk a little faster)
+    const double walk = (two ? t : near + 0.8 * (t - near)) * (n_q < 32 ? (d64 ? 0.93 : 0.75) : 1.0) *
+                        (d64 || gv.kb == 3 ? 1.0 : 0.78);
+    const double work = 1e-5 * t * n * gv.n_q;
+    double here, chain, batch;
+    if (d64) {
+        here = two ? 11.0 + 0.092 * walk : 18.0 + 0.106 * walk;
+        chain = two ? 22.0 + 0.037 * near + 0.44 * n : 19.0 + 0.042 * near + 0.38 * n;
+        batch = two ? 27.0 + 4.95 * work : 22.0 + 3.0 * work;
+    } else {
+        here = two ? 15.0 + 0.181 * walk : 25.0 + 0.236 * walk;
+        chain = two ? 28.0 + 0.070 * near + 0.52 * n : 23.0 + 0.092 * near + 0.38 * n;
+        batch = two ? 35.0 + 8.6 * work : 31.0 + 5.6 * work;
+    }
+    const double there = chain > batch ? chain : batch;
     return here < there;
 }
 
