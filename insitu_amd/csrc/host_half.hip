@@ -9,8 +9,8 @@
 //
 // The projections are fp16 products with fp32 accumulation. A decode step (up
 // to 4 tokens) runs them as one GEMV kernel of this file that streams the
-// weights once and casts its inputs to fp16 itself; a prompt runs them as
-// rocBLAS GEMMs behind a cast kernel. The seam epilogue's float steps follow
+// weights once and casts its inputs to fp16 itself; a prompt runs them on the
+// matrix cores, and a long one as rocBLAS GEMMs behind a cast kernel. The seam epilogue's float steps follow
 // numpy's float64 arithmetic operation by operation (no fused multiply-add), so
 // that for the same fp32 projections the wire rows are the reference's integers
 // exactly. Only the projections' summation order differs from a CPU BLAS.
@@ -40,6 +40,10 @@ __global__ void fixed_to_f16_kernel(const int32_t *__restrict__ x, _Float16 *__r
     if (i < n) y[i] = (_Float16)((double)x[i] * scale);
 }
 
+// The same for Q16, eight values a lane (n a multiple of 8, x 16-byte aligned); q16_to_f16f equals
+// the float64 route.
+__global__ void q16_to_f16x8_kernel(const int32_t *__restrict__ x, _Float16 *__restrict__ y, int64_t n);
+
 // y[r][c] += bias[c] in fp32 (ops/project.py:45-46).
 __global__ void add_bias_kernel(float *__restrict__ y, const float *__restrict__ bias, int64_t rows,
                                 int32_t cols) {
@@ -52,6 +56,9 @@ __global__ void add_bias_kernel(float *__restrict__ y, const float *__restrict__
 // one rounding (fmaf). fp16(x) from fp32 (FIXED = false) or from Q(frac) int32 through
 // float64 (FIXED = true, one rounding, kernel.py:354 to_float).
 constexpr int GEMV_N = 4;
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // fp16(x / 2^16) for int32 x, rounded to nearest even, in integer steps: |x| rounded to 11
 // significant bits (half to even), then scaled, which is exact in fp32 and in fp16 (|x| / 2^16
@@ -176,6 +183,121 @@ __global__ __launch_bounds__(256) void gemv_f16_rows_kernel(
         if (t < n && row < out_f) {
             const float v = (part[0][r][t] + part[1][r][t]) + (part[2][r][t] + part[3][r][t]);
             y[(int64_t)t * out_f + row] = bias ? v + bias[row] : v;
+        }
+    }
+}
+
+__global__ void q16_to_f16x8_kernel(const int32_t *__restrict__ x, _Float16 *__restrict__ y, int64_t n) {
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+    if (i >= n) return;
+    const int4 a = *(const int4 *)(x + i), b = *(const int4 *)(x + i + 4);
+    const int32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    f16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (_Float16)q16_to_f16f(v[e]);
+    *(f16x8 *)(y + i) = o;
+}
+
+// A prompt's projection on the matrix cores: y (n, out_f) = fp16(x) (n, in_f) . W^T (+ bias), sums in
+// fp32. XT = float: x is rounded to fp16 on its way into LDS, so that no cast launch goes before;
+// XT = _Float16: x as it is (a Q16 output is cast once, not once for each tile of W). A workgroup's
+// four waves take 32 NI outputs x 32 NJ tokens, 128 channels a step, with the next step's rows in
+// flight while this one is multiplied (two LDS buffers, one barrier a step; rows 272 bytes apart, so
+// that the 16 rows of an operand read start on 16 different bank quads). Rows past the end are read
+// as the last one and not stored; channels past the end are zeros. Workgroup i runs on XCD i % 8: an XCD takes every
+// 8th group of output rows over all token groups, so that it reads its share of W once.
+template <int NI, int NJ, typename XT>
+__global__ __launch_bounds__(256) void gemm_f16_kernel(const uint16_t *__restrict__ w, int32_t out_f, int32_t in_f,
+                                                       const XT *__restrict__ x, int64_t n, const float *__restrict__ bias,
+                                                       float *__restrict__ y, int32_t tok_groups) {
+    constexpr int BN = 32 * NI, BM = 32 * NJ, BK = 128, PITCH = BK + 8;
+    __shared__ alignas(16) uint16_t ws[2][BN][PITCH];
+    __shared__ alignas(16) uint16_t xs[2][BM][PITCH];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int i8 = blockIdx.x / 8;
+    const int64_t n0 = (int64_t)((int)(blockIdx.x % 8) + 8 * (i8 / tok_groups)) * BN, m0 = (int64_t)(i8 % tok_groups) * BM;
+    if (n0 >= out_f) return;
+    // loads: 16 lanes a row, 8 channels each
+    const int lr = tid >> 4, lk = (tid & 15) * 8;
+    const uint16_t *wp[2 * NI];
+    const XT *xp[2 * NJ];
+#pragma unroll
+    for (int i = 0; i < 2 * NI; ++i) {
+        const int64_t r = n0 + lr + 16 * i;
+        wp[i] = w + (r < out_f ? r : out_f - 1) * in_f;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * NJ; ++i) {
+        const int64_t r = m0 + lr + 16 * i;
+        xp[i] = x + (r < n ? r : n - 1) * in_f;
+    }
+    uint4 wr[2 * NI];
+    constexpr int XQ = sizeof(XT) == 4 ? 2 : 1;
+    uint4 xr[2 * NJ][XQ];
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        const int k = k0 + lk;
+        const bool in = k < in_f;                          // (in_f is a multiple of 8)
+#pragma unroll
+        for (int i = 0; i < 2 * NI; ++i) wr[i] = in ? *(const uint4 *)(wp[i] + k) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2 * NJ; ++i)
+#pragma unroll
+            for (int u = 0; u < XQ; ++u) xr[i][u] = in ? *((const uint4 *)(xp[i] + k) + u) : make_uint4(0, 0, 0, 0);
+    };
+    auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2 * NI; ++i) *(uint4 *)&ws[b][lr + 16 * i][lk] = wr[i];
+#pragma unroll
+        for (int i = 0; i < 2 * NJ; ++i) {
+            if constexpr (XQ == 2) {
+                const uint32_t v[8] = {xr[i][0].x, xr[i][0].y, xr[i][0].z, xr[i][0].w,
+                                       xr[i][1].x, xr[i][1].y, xr[i][1].z, xr[i][1].w};
+                f16x8 h;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) h[e] = (_Float16)__builtin_bit_cast(float, v[e]);
+                *(f16x8 *)&xs[b][lr + 16 * i][lk] = h;
+            } else {
+                *(uint4 *)&xs[b][lr + 16 * i][lk] = xr[i][0];
+            }
+        }
+    };
+    f32x4 acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int ro = 16 * NI * (wv & 1) + (lane & 15), co = 16 * NJ * (wv >> 1) + (lane & 15), kq = (lane >> 4) * 8;
+    const int steps = (in_f + BK - 1) / BK;
+    load(0);
+    for (int st = 0; st < steps; ++st) {
+        const int b = st & 1;
+        store(b);
+        if (st + 1 < steps) load((st + 1) * BK);
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < BK; ks += 32) {
+            f16x8 a[NI], c[NJ];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) a[i] = *(const f16x8 *)&ws[b][ro + 16 * i][ks + kq];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) c[j] = *(const f16x8 *)&xs[b][co + 16 * j][ks + kq];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], c[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // lane = (token, 4 consecutive outputs)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int64_t o = n0 + 16 * NI * (wv & 1) + 16 * i + 4 * (lane >> 4);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int64_t t = m0 + co + 16 * j;
+            if (t >= n) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (o + e < out_f) y[t * out_f + o + e] = bias ? acc[i][j][e] + bias[o + e] : acc[i][j][e];
         }
     }
 }
@@ -346,6 +468,32 @@ bool gemv_fits(int64_t n, int32_t in_f) {
     return n <= GEMV_N && in_f % 8 == 0;
 }
 
+// The prompt's projections on gemm_f16_kernel: 16-byte loads, so channels in eights and aligned rows;
+// up to 2^31 multiply-adds. rocBLAS takes 26 to 28 us a call whatever the size up to there (its call
+// and the cast's launch), and its tiles are the faster ones beyond. Here / there, us, 2,048 -> 3,072
+// from fp32: 5 to 64 tokens 9/27, 256 16/27, 333 24/27, 700 39/27; 2,048 -> 2,048 from Q16: 64 tokens
+// 13/27, 512 20/26, 700 28/26; 4,096 -> 6,144: 5 tokens 19/27, 64 21/27, 128 27/27, 256 43/40.
+bool gemm_fits(const void *w, const void *x, int64_t n, int32_t out_f, int32_t in_f) {
+    return in_f % 8 == 0 && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 && n <= (int64_t(1) << 31) / out_f / in_f;
+}
+
+template <typename XT>
+int gemm(insitu_ctx *c, const uint16_t *w, int32_t out_f, int32_t in_f, const XT *x, int64_t n, const float *bias, float *y) {
+    // 64 x 64 tiles where they give every CU a workgroup, else 32 x 32 (2,048 -> 2,048, 512 tokens: 20.1 us,
+    // 23.6 in 32 x 32; 2,048 -> 3,072, 128 tokens in 32 x 32: 11.9)
+    const bool big = ((n + 63) / 64) * (((int64_t)out_f + 63) / 64) >= 256;
+    const int bt = big ? 64 : 32;
+    const int64_t toks = (n + bt - 1) / bt, outs = ((int64_t)out_f + bt - 1) / bt, grid = (outs + 7) / 8 * 8 * toks;
+    if (big)
+        hipLaunchKernelGGL((gemm_f16_kernel<2, 2, XT>), dim3((unsigned)grid), dim3(256), 0, ctx_stream(c), w, out_f, in_f, x, n,
+                           bias, y, (int32_t)toks);
+    else
+        hipLaunchKernelGGL((gemm_f16_kernel<1, 1, XT>), dim3((unsigned)grid), dim3(256), 0, ctx_stream(c), w, out_f, in_f, x, n,
+                           bias, y, (int32_t)toks);
+    HIP_TRY(hipGetLastError(), "projection");
+    return INSITU_OK;
+}
+
 template <bool FIXED>
 int gemv(insitu_ctx *c, const uint16_t *w, int32_t out_f, int32_t in_f, const void *x, int64_t n, double fscale,
          const float *bias, float *y) {
@@ -409,6 +557,7 @@ int insitu_project(insitu_ctx *c, const uint16_t *w, int32_t out_f, int32_t in_f
     if (n == 0) return INSITU_OK;
     HIP_TRY(hipSetDevice(ctx_device(c)), "hipSetDevice");
     if (gemv_fits(n, in_f)) return gemv<false>(c, w, out_f, in_f, x, n, 0.0, bias, y);
+    if (gemm_fits(w, x, n, out_f, in_f)) return gemm(c, w, out_f, in_f, x, n, bias, y);
     int rc = ensure_x16(c, (size_t)n * in_f);
     if (rc) return rc;
     Blas &b = blas_of(c);
@@ -490,9 +639,14 @@ int insitu_output_projection(insitu_ctx *c, const int32_t *out, int64_t n, int32
     if (rc) return rc;
     Blas &b = blas_of(c);
     const int64_t nx = n * width;
-    hipLaunchKernelGGL(fixed_to_f16_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, ctx_stream(c), out,
-                       b.x16, nx, std::ldexp(1.0, -frac));
+    if (frac == 16 && nx % 8 == 0 && ((uintptr_t)out & 15) == 0)
+        hipLaunchKernelGGL(q16_to_f16x8_kernel, dim3((unsigned)((nx / 8 + 255) / 256)), dim3(256), 0, ctx_stream(c), out,
+                           b.x16, nx);
+    else
+        hipLaunchKernelGGL(fixed_to_f16_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, ctx_stream(c), out,
+                           b.x16, nx, std::ldexp(1.0, -frac));
     HIP_TRY(hipGetLastError(), "fixed to fp16");
+    if (gemm_fits(wo, b.x16, n, hidden, width)) return gemm(c, wo, hidden, width, b.x16, n, bias, y);
     rc = gemm_f16(c, wo, hidden, width, b.x16, n, y);
     if (rc) return rc;
     if (bias) {
