@@ -331,7 +331,9 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     if (own && kvh == 0 && tid == 0) si.len_out[b] = T;
     // a KV head seen as several chains: every one encodes the new row and stores the same words, the
     // first one counts its range errors
-    const bool row_owner = (kvh & ((1 << g.kv_shift) - 1)) == 0;
+    // (4-bit keys come in chains of their own: step_supported)
+    const int kv_shift = KB == 4 ? 0 : g.kv_shift;
+    const bool row_owner = (kvh & ((1 << kv_shift) - 1)) == 0;
     const int score_shift = CENT_FRAC + g.norm_frac;
     const uint8_t *hb = plane_ptr(g, b, kvh, 0);
 
@@ -344,7 +346,7 @@ __global__ void __launch_bounds__(NT, 1) step_kernel(Geom g, const Tables *__res
     // later load waits for every earlier one.
     const int32_t *xsrc = wv < G ? si.qw + ((int64_t)b * g.n_q + kvh * G + wv) * D
                                  : (wv == G + 1 ? si.vw : si.kw) +
-                                       ((int64_t)b * (g.n_kv >> g.kv_shift) + (kvh >> g.kv_shift)) * D;
+                                       ((int64_t)b * (g.n_kv >> kv_shift) + (kvh >> kv_shift)) * D;
     const int32_t xv = xsrc[lane];
     // the new token's encoder: lane i < 2^bits - 1 of wave G (keys) and G + 1 (values) holds
     // boundary i (quantize.py:183-196)
@@ -1733,7 +1735,7 @@ bool step_supported(const Geom &g, int64_t capacity) {
     using namespace stepk;
     const int kbytes = g.d * g.kb / 8;
     const int kpl = kbytes / 16 + (kbytes % 16) / 8;
-    return g.d == D && g.G == G && (g.kb == 4 || g.kb == 3) && g.vb == 2 && g.gq == 0 && g.n_planes == kpl + 2 &&
+    return g.d == D && g.G == G && ((g.kb == 4 && g.kv_shift == 0) || g.kb == 3) && g.vb == 2 && g.gq == 0 && g.n_planes == kpl + 2 &&
            (capacity + CHUNK - 1) / CHUNK <= HMAX && g.norm_frac == 9;
 }
 
