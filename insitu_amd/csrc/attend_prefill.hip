@@ -148,7 +148,8 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
 
     // -- tables, and each row's query digits -------------------------------------------------
     if (tid == 0) {
-        S.rerun = 0;
+        // (not in the wide walk: a wave of this workgroup may still be about to read it there)
+        if constexpr (!WIDE) S.rerun = 0;
         S.events = S.sovf = S.rerr = S.fallbacks = S.mabs = S.macc = 0;
     }
     const int kb = g.kb, vb = g.vb;
@@ -724,6 +725,8 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
         sweep(std::integral_constant<Pass, ONLINE>{});
     }
     if constexpr (!WIDE) {
+        // From this barrier on nothing writes the flag, so that the whole workgroup takes the one way
+        // or the other; the wide walk writes nothing before its first barrier that is read here.
         if (over && valid) S.rerun = 1;
         __syncthreads();
         if (S.rerun) return true;

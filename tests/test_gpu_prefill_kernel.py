@@ -36,10 +36,10 @@ def _run(ctx, fmt, base, n, q, k, v, mode, serial=0):
     host = Cache(N_KV, base + n, f)
     host.append_rotated(k, v)
     fn = native.attend_online if mode == "online" else native.attend_two_pass
-    sts = []
+    sts, views = [], [host.view(h) for h in range(N_KV)]
     for i in range(n):
         for h in range(N_KV):
-            want, s = fn(q[i, G * h:G * h + G], host.view(h).select(slice(0, base + i + 1)), f)
+            want, s = fn(q[i, G * h:G * h + G], views[h].select(slice(0, base + i + 1)), f)
             np.testing.assert_array_equal(out[i, G * h:G * h + G], want, err_msg=f"query {i} head {h}")
             sts.append(s)
     assert st.n_tokens == base + n
@@ -79,6 +79,24 @@ def test_large_values(ctx, fmt, mode, q_scale, kv_scale):
     base, n = 21, 40
     q, k, v = _inputs(7, fmt, base, n, q_scale, kv_scale)
     _run(ctx, fmt, base, n, q, k, v, mode, serial=0 if kv_scale < 1 << 22 else None)
+
+
+@pytest.mark.parametrize("fmt,waves", [((64, 4, 2, 4), 4), ((128, 3, 3, 4), 8)])
+@pytest.mark.parametrize("mode", ["online", "two_pass"])
+@pytest.mark.parametrize("q_wide,q_scale,kv_scale", [(1 << 24, 8192, 65536), (1 << 21, 1 << 10, 1 << 21)])
+def test_one_wave_sends_its_workgroup_to_int64_scores(ctx, fmt, waves, mode, q_wide, q_scale, kv_scale):
+    """One row of a workgroup needs int64 scores (its fourth digit; products past 32 bits), another
+    wave's in each workgroup and none's in every ninth: all its waves start again together."""
+    per_wave = 16 // fmt[3]                            # queries
+    n = 40 * waves * per_wave
+    q, k, v = _inputs(11, fmt, 0, n, q_scale, kv_scale)
+    v = v * 65536 // kv_scale                          # no accumulator near its clamp
+    for b in range(40):
+        if b % 9 != 8:
+            row = q[(b * waves + b % waves) * per_wave + b % per_wave, b % (N_KV * fmt[3])]
+            row[:] = q_wide
+            row[::3] = -q_wide
+    _run(ctx, fmt, 0, n, q, k, v, mode)
 
 
 @pytest.mark.parametrize("fmt", [(64, 4, 2, 4), (128, 3, 3, 4)])
