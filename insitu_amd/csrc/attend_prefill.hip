@@ -345,7 +345,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     // -- the walk ------------------------------------------------------------------------
     SC m = LO, smin = 0;
     v4i acc[C::CT];                                    // lane = (row, 4 channels of each tile)
-    uint32_t lp = 0;                                   // this lane's part of the denominator since the last event
+    uint32_t lp = 0;                                   // this lane's part of the denominator since the last event or fold
     uint64_t l64 = 0;                                  // the row's denominator up to there
     uint32_t n_events = 0, n_sovf = 0;
     float bsum = 0.0f;                                 // bound of |acc| over the wave's rows
@@ -379,6 +379,14 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             const uint32_t w = (uint32_t)hi - (uint32_t)lo;
             return w < delta_max ? w : delta_max;
         }
+    };
+
+    // the row's denominator, in its four lanes
+    auto denominator = [&]() __attribute__((always_inline)) -> uint64_t {
+        uint64_t tot = lp;
+        tot += shfl_s<uint64_t>(tot, lane ^ 16);
+        tot += shfl_s<uint64_t>(tot, lane ^ 32);
+        return l64 + tot;
     };
 
     // acc += the terms in A: the sums of the highest digits first, each carried into the next
@@ -667,11 +675,9 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
                 for (int i = 0; i < 4; ++i) acc[c][i] = (int32_t)(((int64_t)acc[c][i] * f) >> PROB_FRAC);
                 __builtin_amdgcn_sched_barrier(0);     // few products in flight: registers
             }
-            uint64_t tot = lp;
-            tot += shfl_s<uint64_t>(tot, lane ^ 16);
-            tot += shfl_s<uint64_t>(tot, lane ^ 32);
+            const uint64_t l = denominator();
             if (has) {
-                l64 = ((l64 + tot) * (uint64_t)f) >> PROB_FRAC;
+                l64 = (l * (uint64_t)f) >> PROB_FRAC;
                 lp = 0;
             }
         }
@@ -711,6 +717,11 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             const int32_t ts = s * C::ST;
             for (int tl = 0; tl < C::NT && ts + tl * 16 < wmax; ++tl)
                 tile(passc, bf, tl, ts + tl * 16, ts + tl * 16 + 16 > wmin, check, tight);
+            // a stage adds at most 16 tokens of 2^15 to a lane's 32 bits
+            if (P != MAXONLY && (s & 4095) == 4095) {
+                l64 = denominator();
+                lp = 0;
+            }
         }
         __syncthreads();
     };
@@ -734,10 +745,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
 
     // -- finalize --------------------------------------------------------------------------
     {
-        uint64_t tot = lp;
-        tot += shfl_s<uint64_t>(tot, lane ^ 16);
-        tot += shfl_s<uint64_t>(tot, lane ^ 32);
-        const Recip rc = reciprocal((int64_t)(l64 + tot));
+        const Recip rc = reciprocal((int64_t)denominator());
         const bool mine = valid && !bad;
         const int64_t at = ((rowc / G) * g.n_q + (int64_t)kvh * G + rowc % G) * D;
         int64_t macc = 0;

@@ -115,6 +115,34 @@ def test_clamped_accumulators_and_wide_terms(ctx, fmt, mode):
     _run(ctx, fmt, 300, n, q, k[:300 + n], v[:300 + n], mode, serial=0)
 
 
+@pytest.mark.parametrize("fmt", [(64, 4, 2, 4), (64, 2, 3, 1), (128, 3, 3, 2)])
+@pytest.mark.parametrize("mode", ["online", "two_pass"])
+def test_denominators_past_32_bits_a_lane(ctx, fmt, mode):
+    """Equal and nearly equal scores over more than 2^19 rows: a lane's share of the denominator, four
+    rows of 16 at 2^15 each, passes 2^32."""
+    from insitu_amd.attention import CompressedAttention
+    d, kb, vb, G = fmt
+    f = Format(d=d, key_bits=kb, value_bits=vb)
+    T, n, tile = (1 << 19) + 700, 3, 4096
+    q, k, v = _inputs(5, fmt, tile - n, n, 16, 8192)
+    q[0] = 0
+    c, host = _cache(ctx, T, *fmt), Cache(N_KV, tile, f)
+    host.append_rotated(k, v)
+    for t in range(0, T, tile):
+        c.append_rotated(k[:T - t], v[:T - t])
+    out, st = CompressedAttention(c).attend_prefill(q, T - n, mode)
+    out = out.cpu().numpy()
+    fn = native.attend_online if mode == "online" else native.attend_two_pass
+    for h in range(N_KV):
+        kv = host.view(h)
+        rep = lambda a: np.concatenate([a] * (T // tile + 1))
+        kv = type(kv)(rep(kv.k_idx), rep(kv.k_norm), rep(kv.v_idx), rep(kv.v_norm))
+        for i in range(n):
+            want, _ = fn(q[i, G * h:G * h + G], kv.select(slice(0, T - n + i + 1)), f)
+            np.testing.assert_array_equal(out[i, G * h:G * h + G], want, err_msg=f"query {i} head {h}")
+    assert st.serial_fallbacks == 0 and st.n_tokens == T
+
+
 def test_range_errors_and_rows_past_exact_scores(ctx):
     """Queries past the rotated range are counted; a row whose scores may not be exact (a value
     of 2^30) takes the reference loop, alone."""
