@@ -555,7 +555,7 @@ int insitu_cache_create(insitu_ctx *c, const insitu_cache_desc *desc, insitu_cac
         k->gpad = k->chunked;
     }
     k->step = step_supported(step_geom(k, g), desc->capacity);
-    k->split = split_supported(g, desc->capacity);
+    k->split = split_supported(g, t, desc->capacity);
     if (e == hipSuccess && (k->chunked || k->scan || k->step || k->split)) {
         size_t nb = k->split ? split_scratch_bytes(g, desc->capacity) : 0;
         if (k->step) {

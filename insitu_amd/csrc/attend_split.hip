@@ -26,6 +26,9 @@
 // tokens at d = 64, 8 KV heads: 23.2 us (75.0 as a write, a maximum and a summing launch of 1,024
 // tokens a workgroup in fp64). Beyond, the matrix products and the digits' extraction: a flat softmax
 // over 16 x 32,768 tokens 213 us (833), of 131,072 tokens 98 us (281).
+#include <algorithm>
+#include <cstdlib>
+
 #include "digits.h"
 #include "query.h"
 #include "row_codec.h"
@@ -757,8 +760,12 @@ size_t carve(const Geom &g, int64_t capacity, uint8_t *p, Scratch *sc, size_t *f
 
 }  // namespace sp
 
-bool split_supported(const Geom &g, int64_t capacity) {
-    return (g.d == 64 || g.d == 128) && g.kb >= 2 && g.kb <= 4 && g.vb >= 1 && g.vb <= 3 && g.norm_frac == 9 &&
+// (A term t = floor(v_norm p c / 2^23) is at most 128 |c|; its digits are read from the fp64 sum while
+// that stays below 2^29, i.e. t + 0x808080 below 2^27. Wider value centroids take the chunked attend.)
+bool split_supported(const Geom &g, const Tables &th, int64_t capacity) {
+    int64_t vmax = 0;
+    for (int i = 0; i < (1 << g.vb); ++i) vmax = std::max<int64_t>(vmax, std::llabs(th.vc[i]));
+    return 128 * vmax + 0x808080 < (int64_t(1) << 27) && (g.d == 64 || g.d == 128) && g.kb >= 2 && g.kb <= 4 && g.vb >= 1 && g.vb <= 3 && g.norm_frac == 9 &&
            g.G >= 1 && g.G <= 8 && g.kv_shift == 0 && g.gq == 0 &&
            capacity <= (int64_t)sp::MAXWG * sp::W * sp::MAXU * sp::BT;
 }

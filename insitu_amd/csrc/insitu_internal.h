@@ -323,7 +323,7 @@ hipError_t launch_step_write(hipStream_t s, const Geom &g, const Tables *t, cons
 // The two-pass attend in two launches (attend_split.hip): one query a sequence, or with step the whole decode step
 // (len the lengths before it); longest: the longest sequence, the new token
 // included.
-bool split_supported(const Geom &g, int64_t capacity);
+bool split_supported(const Geom &g, const Tables &host_tabs, int64_t capacity);
 size_t split_scratch_bytes(const Geom &g, int64_t capacity);
 hipError_t launch_attend_split(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,
                                const int64_t *len, ChunkScratch &cs, int64_t longest, const StepIn *step, LaunchEv ev,

@@ -102,6 +102,51 @@ def test_sums_that_clamp(ctx, fmt):
     assert _attend(ctx, fmt, (300,), q, k, v).acc_overflows == 0
 
 
+@pytest.mark.parametrize("d,kb,vb", [(64, 4, 2), (64, 3, 3), (128, 3, 3), (128, 4, 2)])
+@pytest.mark.parametrize("c_max,taken", [(982_782, True), (982_783, False), ((1 << 20) - 1, False)])
+def test_value_centroids_up_to_20_bits(ctx, monkeypatch, d, kb, vb, c_max, taken):
+    """Terms up to the digits' limit with the largest norm and p = 1; a codebook past it is refused by
+    the split attend, and the automatic choice gives the oracle's outputs all the same."""
+    import dataclasses
+
+    from insitu_amd import QuantConfig, _lib
+    from insitu_amd.attention import CompressedAttention
+    from insitu_amd.cache import Codebook, CompressedCache
+    n = 1 << vb
+    vc = np.rint(np.linspace(-1, 1, n) * c_max).astype(np.int64)
+
+    class Wide(Format):
+        def codebooks(self):
+            k_c, k_b, _, v_b = super().codebooks()
+            return k_c, k_b, vc, v_b
+
+    build = Codebook.build
+    books = iter([None, vc])                          # CompressedCache builds the key's first
+    monkeypatch.setattr(Codebook, "build", staticmethod(
+        lambda *a: build(*a) if (v := next(books)) is None else dataclasses.replace(build(*a), centroids=v)))
+    T, G = 70, 4
+    c = CompressedCache(N_KV, d, T, QuantConfig(key_bits=kb, value_bits=vb), n_q_heads=N_KV * G, ctx=ctx)
+    rng = np.random.default_rng(d + vb)
+    # the largest norm; a quarter of the channels at twice it, in the outermost codes
+    v = np.where(rng.random((T, N_KV, d)) < 0.25, 1 << 24, 0) * rng.choice([-1, 1], (T, N_KV, d))
+    k = _draw(rng, 65536, T, N_KV, d)
+    q = _draw(rng, 8192, 1, N_KV * G, d)
+    q[0, 1:3] = 0                                     # p = 1 throughout
+    f = Wide(d=d, key_bits=kb, value_bits=vb)
+    host = Cache(N_KV, T, f)
+    host.append_rotated(k, v)
+    assert host.view(0).v_norm.max() == 32767 and {0, n - 1} <= set(host.view(0).v_idx.ravel().tolist())
+    c.append_rotated(k, v)
+    a = CompressedAttention(c)
+    for pin in ("auto", "split") if taken else ("auto",):
+        c.pin_kernel(pin)
+        out, st = a.attend(q, "two_pass")
+        _check(out.cpu().numpy(), st, q, [host], f, G, serial=None)
+    if not taken:
+        with pytest.raises(_lib.FormatError, match="EINVAL"):
+            c.pin_kernel("split")
+
+
 def test_range_errors_and_scores_that_may_not_be_exact(ctx):
     """Queries past the rotated range are counted; a head with a value of 2^30 takes the reference
     loop, alone."""
