@@ -390,7 +390,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     };
 
     // acc += the terms in A: the sums of the highest digits first, each carried into the next
-    // product's accumulator. WIDE's terms have a fourth digit, of weight 2^20.
+    // product's accumulator. WIDE's terms have a fourth digit, of weight 2^21.
     auto accumulate = [&](const v4i (&A)[WIDE ? 4 : 3][C::PVK], int bf, int tl) __attribute__((always_inline)) {
         constexpr int GC = 4;                          // channel tiles at a time, to cover the products' latency
 #pragma unroll
@@ -406,7 +406,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
 #pragma unroll
                 for (int k = 0; k < C::PVK; ++k) {
                     t[c] = mma(o[c][k], A[2][k], t[c]);
-                    if constexpr (WIDE) t[c] = mma(o[c][k] << 4, A[3][k], t[c]);
+                    if constexpr (WIDE) t[c] = mma(o[c][k] << 5, A[3][k], t[c]);
                 }
             }
 #pragma unroll
@@ -560,11 +560,11 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
                         uint32_t z[4], d2 = 0, d3 = 0;
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
-                            const int32_t t = (int32_t)floor(wd * vcs[4 * k4 + k]);   // |t| < 2^27
+                            const int32_t t = (int32_t)floor(wd * vcs[4 * k4 + k]);   // |t| < 2^27: top at most 2^11
                             z[k] = ((uint32_t)t + 0x8080u) ^ 0x8080u;
                             const int32_t top = (int32_t)((uint32_t)t + 0x8080u) >> 16;
-                            d2 |= (uint32_t)(top & 15) << (8 * k);
-                            d3 |= ((uint32_t)(top >> 4) & 0xFFu) << (8 * k);
+                            d2 |= (uint32_t)(top & 31) << (8 * k);
+                            d3 |= ((uint32_t)(top >> 5) & 0xFFu) << (8 * k);
                         }
                         const uint32_t a = perm(z[1], z[0], 0x05010400u), b = perm(z[3], z[2], 0x05010400u);
                         A[0][kbk][dw] = (int)perm(b, a, 0x05040100u);

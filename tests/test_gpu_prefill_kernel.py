@@ -115,6 +115,48 @@ def test_clamped_accumulators_and_wide_terms(ctx, fmt, mode):
     _run(ctx, fmt, 300, n, q, k[:300 + n], v[:300 + n], mode, serial=0)
 
 
+@pytest.mark.parametrize("fmt", [(64, 4, 2, 4), (64, 2, 3, 1), (128, 3, 3, 2), (128, 4, 2, 8)])
+@pytest.mark.parametrize("mode", ["online", "two_pass"])
+def test_value_centroids_at_20_bits(ctx, monkeypatch, fmt, mode):
+    """The largest terms: centroids of 2^20 - 1, the largest norm, p = 1. The first 16 rows' sums fit the
+    accumulator's bound, the later rows take the reference loop."""
+    import dataclasses
+
+    from insitu_amd.attention import CompressedAttention
+    from insitu_amd.cache import Codebook
+    d, kb, vb, G = fmt
+    vc = np.rint(np.linspace(-1, 1, 1 << vb) * ((1 << 20) - 1)).astype(np.int64)
+
+    class Wide(Format):
+        def codebooks(self):
+            k_c, k_b, _, v_b = super().codebooks()
+            return k_c, k_b, vc, v_b
+
+    build = Codebook.build
+    books = iter([None, vc])                          # CompressedCache builds the key's first
+    monkeypatch.setattr(Codebook, "build", staticmethod(
+        lambda *a: build(*a) if (v := next(books)) is None else dataclasses.replace(build(*a), centroids=v)))
+    n = 24
+    c = _cache(ctx, n, *fmt)
+    q, k, v = _inputs(2, fmt, 0, n, 4096, 65536)
+    q[:, ::2] = 0
+    rng = np.random.default_rng(1)
+    v = np.where(rng.random(v.shape) < 0.25, 1 << 24, 0) * rng.choice([-1, 1], v.shape)
+    f = Wide(d=d, key_bits=kb, value_bits=vb)
+    host = Cache(N_KV, n, f)
+    host.append_rotated(k, v)
+    assert host.view(0).v_norm.max() == 32767 and {0, (1 << vb) - 1} <= set(host.view(0).v_idx.ravel().tolist())
+    c.append_rotated(k, v)
+    out, st = CompressedAttention(c).attend_prefill(q, 0, mode)
+    out = out.cpu().numpy()
+    fn = native.attend_online if mode == "online" else native.attend_two_pass
+    for i in range(n):
+        for h in range(N_KV):
+            want, _ = fn(q[i, G * h:G * h + G], host.view(h).select(slice(0, i + 1)), f)
+            np.testing.assert_array_equal(out[i, G * h:G * h + G], want, err_msg=f"query {i} head {h}")
+    assert st.serial_fallbacks < n * N_KV * G
+
+
 @pytest.mark.parametrize("fmt", [(64, 4, 2, 4), (64, 2, 3, 1), (128, 3, 3, 2)])
 @pytest.mark.parametrize("mode", ["online", "two_pass"])
 def test_denominators_past_32_bits_a_lane(ctx, fmt, mode):
