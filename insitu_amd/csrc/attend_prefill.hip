@@ -51,7 +51,8 @@
 namespace insitu {
 namespace pf {
 
-constexpr double TWO55 = 36028797018963968.0;
+// |dot k_norm| below this: floor(dot k_norm / 2^24) is above INT32_MIN, the narrow scores' "none yet"
+constexpr double NARROW_LIMIT = 36028797018963968.0 - 16777216.0;
 constexpr uint32_t LUT_N = LUT_SPAN + 1;               // p by floor index, the last entry 0
 constexpr double TERM_MAGIC = 402653184.0 + 8421504.0; // 1.5 * 2^28 + 0x808080: ulp 2^-24
 constexpr double TERM_LIMIT = 8355711.0;               // 0x7F7F7F: three balanced bytes
@@ -465,7 +466,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             }
             if (check) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) over |= (x[i] >> 8) != (int64_t)s[i] && !bad;
+                for (int i = 0; i < 4; ++i) over |= ((x[i] >> 8) != (int64_t)s[i] || s[i] == LO) && !bad;
             }
         } else {
             v4i T[NQ + 2];
@@ -698,7 +699,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             __syncthreads();
             if (s + 1 < nst) expand(bf ^ 1, P != MAXONLY);
             // narrow scores fit 32 bits when the largest product does (else they are looked at)
-            const bool check = uni32(!(bq * (double)S.knmax[bf] < TWO55));
+            const bool check = uni32(!(bq * (double)S.knmax[bf] < NARROW_LIMIT));
             // the largest |term| of the stage's tokens, p at most 1, and the floor
             const double term = (double)uni32(S.vnmax[bf]) * 32768.0 * vcmax + 2.0;
             if (!WIDE && term > TERM_LIMIT) over = true;

@@ -81,6 +81,34 @@ def test_large_values(ctx, fmt, mode, q_scale, kv_scale):
     _run(ctx, fmt, base, n, q, k, v, mode, serial=0 if kv_scale < 1 << 22 else None)
 
 
+@pytest.mark.parametrize("mode", ["online", "two_pass"])
+@pytest.mark.parametrize("target", [-(1 << 31), -(1 << 31) + 1])
+def test_scores_at_the_end_of_32_bits(ctx, mode, target):
+    """A first score of -2^31, the narrow scores' mark of a row with no token yet, is an event too."""
+    fmt = (64, 4, 2, 4)
+    d, kb, vb, G = fmt
+    f = Format(d=d, key_bits=kb, value_bits=vb)
+    q, k, v = _inputs(4, fmt, 0, 3, 64, 1 << 21)
+    host = Cache(N_KV, 3, f)
+    host.append_rotated(k, v)
+    kv, kc = host.view(0), f.codebooks()[0]
+    c, kn = kc[kv.k_idx[0].astype(int)], int(kv.k_norm[0])
+    # dot in [target 2^24 / kn, (target + 1) 2^24 / kn): all channels alike, then two channels' steps
+    lo, hi = -((-target << 24) // kn), -((-(target + 1) << 24) // kn)
+    x = (np.sign(c) * (lo // int(np.abs(c).sum()))).astype(np.int64)
+    i, j = np.argmax(c), np.argmin(np.abs(np.abs(c) - 4200))
+    rest = lo - int(x @ c)
+    for s in range(-20000, 20000):
+        t = (rest - s * int(c[j])) // int(c[i]) + 1
+        if lo <= int(x @ c) + s * int(c[j]) + t * int(c[i]) < hi:
+            break
+    x[j] += s
+    x[i] += t
+    assert (int(x @ c) * kn) >> 24 == target and np.abs(x).max() < 0x7F7F7F and i != j
+    q[0, 1] = x
+    _run(ctx, fmt, 0, 3, q, k, v, mode)
+
+
 @pytest.mark.parametrize("fmt,waves", [((64, 4, 2, 4), 4), ((128, 3, 3, 4), 8)])
 @pytest.mark.parametrize("mode", ["online", "two_pass"])
 @pytest.mark.parametrize("q_wide,q_scale,kv_scale", [(1 << 24, 8192, 65536), (1 << 21, 1 << 10, 1 << 21)])
