@@ -305,8 +305,9 @@ enum {
                                         handles the format                                      */
     INSITU_DEBUG_PREFILL = 6         /* the causal attends' kernel: 0 automatic (the prefill kernel
                                         where it handles the format and the queries fill it), 1 the
-                                        decode attends over a virtual batch, 2 the prefill kernel;
-                                        INSITU_EINVAL if it does not handle the cache            */
+                                        decode attends over a virtual batch, 2 the prefill kernel
+                                        for up to 2^27 rows; INSITU_EINVAL if it does not handle
+                                        the cache                                               */
 };
 int insitu_cache_debug(insitu_cache *cache, int32_t what, int64_t value);
 /* The statistics the cache's kernels have gathered since they were last cleared (an
@@ -323,6 +324,11 @@ int insitu_cache_stats(insitu_cache *cache, insitu_stats *stats_host);
  * slot id limit. */
 int insitu_debug_scratch_layout(int32_t kernel, int64_t capacity, int32_t batch, int32_t n_kv, int32_t d,
                                 int64_t *facts, int32_t n);
+/* Whether a causal attend of n_q queries behind base rows runs on the prefill kernel (1) when
+ * nothing is pinned, computed on the host without a GPU; chunked: the chunked attend handles the
+ * cache. */
+int insitu_debug_prefill_rule(const insitu_format *fmt, int32_t n_q_heads, int32_t n_kv_heads, int32_t chunked,
+                              int64_t base, int64_t n_q, int32_t mode, int32_t *prefill_kernel);
 
 /* Message of the last failing call on this thread. */
 const char *insitu_last_error(void);

@@ -35,7 +35,7 @@ EXPORTS = (
     "insitu_output_projection", "insitu_read_rows", "insitu_load_rows", "insitu_read_image",
     "insitu_load_image", "insitu_probe_read", "insitu_probe_empty", "insitu_cache_debug",
     "insitu_cache_stats",
-    "insitu_debug_scratch_layout", "insitu_last_error",
+    "insitu_debug_scratch_layout", "insitu_debug_prefill_rule", "insitu_last_error",
 )
 
 
@@ -141,6 +141,7 @@ def load(path: str | None = None):
         "insitu_cache_debug": (i32, [vp, i32, i64]),
         "insitu_cache_stats": (i32, [vp, P(Stats)]),
         "insitu_debug_scratch_layout": (i32, [i32, i64, i32, i32, i32, P(i64), i32]),
+        "insitu_debug_prefill_rule": (i32, [P(Format), i32, i32, i32, i64, i64, i32, P(i32)]),
         "insitu_last_error": (ctypes.c_char_p, []),
     }
     for name, (res, args) in sig.items():

@@ -876,11 +876,12 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 // 0.5 % longer than the better kernel in the mean of them, 1.3 times as long at the worst. E.g. here /
 // there us, d = 64, online: 16 queries of 64 rows 25/27, 256 rows 50/35, 2,048 rows 220/68; 128 of
 // 256 rows 50/83, of 2,048 rows 221/273; d = 128, 3/3 bits: 64 of 512 rows 157/96, 192 263/408 of 1,024.
-static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
-    if (mode == INSITU_SERIAL || !prefill_supported(gv) || k->prefill_path == 1) return false;
-    if (k->prefill_path == 2) return true;
-    if (k->path != 0 && k->path != 4) return false;
-    if (!k->chunked) return true;           // else token by token
+static bool prefill_kernel_takes(const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
+    return mode != INSITU_SERIAL && prefill_supported(gv) && base + n_q <= PREFILL_MAX_ROWS;
+}
+static bool prefill_rule(const Geom &gv, bool chunked, int64_t base, int64_t n_q, int32_t mode) {
+    if (!prefill_kernel_takes(gv, base, n_q, mode)) return false;
+    if (!chunked) return true;              // else token by token
     const bool two = mode == INSITU_TWO_PASS, d64 = gv.d == 64;
     const double t = (double)(base + n_q), near = t < 1024.0 ? t : 1024.0, n = (double)n_q;
     // (3-bit codes at d = 128 take most to load and widen; few waves walk a little faster)
@@ -899,6 +900,12 @@ static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t ba
     }
     const double there = chain > batch ? chain : batch;
     return here < there;
+}
+static bool use_prefill_kernel(const insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
+    if (k->prefill_path == 1) return false;
+    if (k->prefill_path == 2) return prefill_kernel_takes(gv, base, n_q, mode);
+    if (k->path != 0 && k->path != 4) return false;
+    return prefill_rule(gv, k->chunked, base, n_q, mode);
 }
 
 static int prefill_kernel_launch(insitu_cache *k, const Geom &gv, int64_t base, int64_t n_q, const int32_t *q,
@@ -1131,6 +1138,25 @@ int insitu_debug_scratch_layout(int32_t kernel, int64_t capacity, int32_t batch,
         insitu::step_layout_facts(g, insitu::step_max_chunks(capacity), facts);
     else
         return fail(INSITU_EINVAL, "kernel: 0 chunked (1,024-token chunks), 1 chunked (512), 2 step (d = 64)");
+    return INSITU_OK;
+}
+
+// Test hook: the automatic choice of a causal attend's kernel, computed on the host (no GPU call).
+int insitu_debug_prefill_rule(const insitu_format *fmt, int32_t n_q_heads, int32_t n_kv_heads, int32_t chunked,
+                              int64_t base, int64_t n_q, int32_t mode, int32_t *prefill_kernel) {
+    std::string why;
+    if (!fmt || !prefill_kernel || n_kv_heads < 1 || n_q_heads < 1 || n_q_heads % n_kv_heads || base < 0 || n_q < 0 ||
+        mode < INSITU_SEQUENTIAL || mode > INSITU_SERIAL || !format_supported(*fmt, why))
+        return fail(INSITU_EINVAL, "bad argument");
+    Geom g{};
+    g.d = fmt->head_dim;
+    g.kb = fmt->key_bits;
+    g.vb = fmt->value_bits;
+    g.norm_frac = fmt->norm_frac;
+    g.n_kv = n_kv_heads;
+    g.n_q = n_q_heads;
+    g.G = g.n_q / g.n_kv;
+    *prefill_kernel = prefill_rule(g, chunked != 0, base, n_q, mode) ? 1 : 0;
     return INSITU_OK;
 }
 

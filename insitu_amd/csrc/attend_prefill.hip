@@ -836,6 +836,7 @@ bool prefill_supported(const Geom &g) {
 hipError_t launch_attend_prefill(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,
                                  int64_t base, int64_t n_q, int two_pass, LaunchEv ev, DevStats *st) {
     if (n_q <= 0) return hipSuccess;
+    if (base < 0 || base + n_q > PREFILL_MAX_ROWS) return hipErrorInvalidValue;
     if (g.d == 64) {
         // A grid that fills the chip runs three workgroups a CU (32-token stages: 42 KB of LDS, 168
         // VGPRs); a smaller one has a CU each, and longer stages amortise their barriers.

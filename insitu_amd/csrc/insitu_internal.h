@@ -329,7 +329,9 @@ hipError_t launch_attend_split(hipStream_t s, const Geom &g, const Tables *t, co
                                const int64_t *len, ChunkScratch &cs, int64_t longest, const StepIn *step, LaunchEv ev,
                                DevStats *st);
 // The prefill attend on matrix cores (attend_prefill.hip): query i of n_q (rows of q, (n_q,
-// g.n_q, d)) over rows 0 .. base + i of the sequence at g.base; no scratch, one launch.
+// g.n_q, d)) over rows 0 .. base + i of the sequence at g.base; no scratch, one launch. base + n_q
+// is at most PREFILL_MAX_ROWS: a row's byte offset in a plane (16 a row) is an int32 there.
+constexpr int64_t PREFILL_MAX_ROWS = int64_t(1) << 27;
 bool prefill_supported(const Geom &g);
 hipError_t launch_attend_prefill(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,
                                  int64_t base, int64_t n_q, int two_pass, LaunchEv ev, DevStats *st);

@@ -287,6 +287,36 @@ def test_scratch_layout_invariants(kernel):
     assert "total > NSEG" in src
 
 
+def _prefill_rule(lib, base, n_q, mode, d=64, kb=4, vb=2, n_q_heads=32, n_kv=8, chunked=1):
+    from insitu_amd import _lib
+    f = _lib.Format(head_dim=d, key_bits=kb, value_bits=vb, norm_bits=16, norm_frac=9, qk_frac=16, qk_width=24,
+                    centroid_frac=15, acc_frac=16, acc_width=32, score_width=48, prob_frac=15, exp_lut_bits=8)
+    out = ctypes.c_int32(-1)
+    rc = lib.insitu_debug_prefill_rule(ctypes.byref(f), n_q_heads, n_kv, chunked, base, n_q, _lib.MODES[mode],
+                                       ctypes.byref(out))
+    assert rc == 0, lib.insitu_last_error()
+    return out.value
+
+
+def test_causal_attends_past_the_prefill_kernels_rows():
+    """Its row offsets, 16 bytes a row, are 32-bit: past 2^27 rows a causal attend runs on the general
+    kernels (computed on the host, no GPU call), as do the formats it does not take."""
+    from insitu_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.load()
+    rows = (2**31 - 1 - 15) // 16 + 1                  # the last row's 16 bytes end below 2^31
+    assert rows == 1 << 27
+    for mode in ("online", "two_pass", "split"):
+        for n in (1, 4096):
+            assert _prefill_rule(lib, rows - n, n, mode, chunked=0) == 1
+            assert _prefill_rule(lib, rows - n + 1, n, mode, chunked=0) == 0
+            assert _prefill_rule(lib, 2 * rows, n, mode, chunked=0) == 0
+        assert _prefill_rule(lib, 0, 4096, mode) == 1
+        assert _prefill_rule(lib, 0, 4096, mode, kb=5) == 0
+    assert _prefill_rule(lib, 0, 4096, "serial") == 0
+
+
 def test_block_chunk_size_follows_capacity():
     """A block's cache takes 512-token chunks only while the chunked attend's chunk limit
     holds them; past 262,144 tokens it keeps 1,024-token chunks (and the chunked path)."""
