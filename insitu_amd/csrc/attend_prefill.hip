@@ -58,6 +58,11 @@ constexpr double TERM_MAGIC = 402653184.0 + 8421504.0; // 1.5 * 2^28 + 0x808080:
 constexpr double TERM_LIMIT = 8355711.0;               // 0x7F7F7F: three balanced bytes
 constexpr float ACC_BOUND = 2147483520.0f;             // the largest float below 2^31
 
+// 16 bytes of a 4-byte aligned address: query rows, outputs and narrow planes
+struct __attribute__((aligned(4))) u128 {
+    uint32_t x, y, z, w;
+};
+
 enum Pass { MAXONLY = 0, FIXEDMAX = 1, ONLINE = 2 };
 
 // Bytes b of four words, as the four dwords of bytes 0, 1, 2, 3.
@@ -193,8 +198,8 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             uint32_t z[16];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int4 v = valid ? *(const int4 *)(qp + b * 64 + 4 * i) : make_int4(0, 0, 0, 0);
-                const int32_t x[4] = {v.x, v.y, v.z, v.w};
+                const u128 v = valid ? *(const u128 *)(qp + b * 64 + 4 * i) : u128{0, 0, 0, 0};
+                const int32_t x[4] = {(int32_t)v.x, (int32_t)v.y, (int32_t)v.z, (int32_t)v.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t ax = x[j] < 0 ? 0u - (uint32_t)x[j] : (uint32_t)x[j];
@@ -237,9 +242,6 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     // -- staging -------------------------------------------------------------------------
     // Plane p of the stage's tokens, 16 bytes a load (a narrower record's tail is the next ones',
     // or the span's padding: a span holds 16 bytes a token).
-    struct __attribute__((aligned(4))) u128 {
-        uint32_t x, y, z, w;
-    };
     u128 rg[C::UNITS];
     const uint8_t *src[C::UNITS];
     int width[C::UNITS];
@@ -752,14 +754,14 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
         int64_t macc = 0;
 #pragma unroll
         for (int c = 0; c < C::CT; ++c) {
-            int32_t o[4];
+            uint32_t o[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int64_t a = acc[c][i], aa = a < 0 ? -a : a;
                 macc = aa > macc ? aa : macc;
-                o[i] = (int32_t)(wmul(a, rc.r) >> rc.shift);
+                o[i] = (uint32_t)(wmul(a, rc.r) >> rc.shift);
             }
-            if (mine) *(int4 *)(out + at + c * 16 + grp * 4) = make_int4(o[0], o[1], o[2], o[3]);
+            if (mine) *(u128 *)(out + at + c * 16 + grp * 4) = u128{o[0], o[1], o[2], o[3]};
         }
         const int64_t mp = (int64_t)m < 0 ? -(int64_t)m : (int64_t)m, mn = -(int64_t)smin;
         const int64_t ev = wave_sum_i64(mine ? n_events : 0), ov = wave_sum_i64(mine ? n_sovf : 0);

@@ -224,6 +224,27 @@ def test_range_errors_and_rows_past_exact_scores(ctx):
     assert st.range_errors == 2
 
 
+@pytest.mark.parametrize("fmt", [(64, 4, 2, 4), (128, 3, 3, 4)])
+def test_rows_at_4_byte_aligned_addresses(ctx, fmt):
+    """q and out as views one int32 into a larger tensor."""
+    import torch
+
+    from insitu_amd.attention import CompressedAttention
+    d, _, _, G = fmt
+    n = 21
+    q, k, v = _inputs(8, fmt, 0, n, 8192, 65536)
+    c = _cache(ctx, n, *fmt)
+    c.append_rotated(k, v)
+    a = CompressedAttention(c)
+    want = a.attend_prefill(q, 0, "online")[0]
+    bufs = [torch.zeros(q.size + 1, dtype=torch.int32, device=ctx.torch_device) for _ in "qo"]
+    q1, o1 = (b[1:].view(q.shape) for b in bufs)
+    q1.copy_(torch.from_numpy(q))
+    assert q1.data_ptr() % 16 == o1.data_ptr() % 16 == 4
+    got = a.attend_prefill(q1, 0, "online", out=o1)[0]
+    assert torch.equal(got, want) and int(bufs[1][0]) == 0
+
+
 @pytest.mark.parametrize("mode", ["online", "two_pass"])
 def test_auto_choice_equals_both_kernels(ctx, mode):
     """The automatic choice and either pinned kernel give the same output, either side of the rule."""
