@@ -1,10 +1,13 @@
 """The chunked attend's matrix-core scores at their edges: every key width, head dimension and
 chunk build, context lengths around the tiles and the halves of a wave, and query values at the
-ends of int32, against the token-by-token kernel."""
+ends of int32, against the token-by-token kernel and, in two-pass mode, oracle/c."""
 
 import numpy as np
 import pytest
 import torch
+
+from oracle import native
+from oracle.quantize import Format
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +39,10 @@ def test_scores_equal_the_token_by_token_kernel(ctx, d, kb, vb, chunk_tokens):
         got = attn.attend(qs, "online", stats=False)[0]
         want = attn.attend(qs, "serial", stats=False)[0]
         assert torch.equal(got, want)
+        out = attn.attend(qs, "two_pass", stats=False)[0].cpu().numpy()
+        q_np = qs.cpu().numpy()
+        for b in range(len(lens)):
+            for h in range(2):
+                kv = cache.view(h, seq=b).host()
+                want = native.attend_two_pass(q_np[b, 4 * h:4 * h + 4], kv, Format(d=d, key_bits=kb, value_bits=vb))[0]
+                np.testing.assert_array_equal(out[b, 4 * h:4 * h + 4], want, err_msg=f"{lens[b]} rows, head {h}")

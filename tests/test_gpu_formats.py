@@ -76,8 +76,9 @@ def test_eight_query_heads_on_the_chunked_attend(ctx, T, kb, vb):
 
 
 def test_eight_query_heads_decode_steps_and_prefill(ctx):
-    """insitu_step (two launches: the write kernel, then the attend) and the causal prefill
-    on a 3b/2b cache with 8 query heads a KV head, against the oracle's step loop."""
+    """insitu_step (the step kernel; pinned to the chunked attend, in test_gpu_general_kernels,
+    two launches) and the causal prefill on a 3b/2b cache with 8 query heads a KV head,
+    against the oracle's step loop."""
     import torch
     from insitu_amd import _lib
     from insitu_amd.attention import CompressedAttention

@@ -929,9 +929,9 @@ def test_prefill_is_the_token_loop(ctx, kb, vb, mode):
 
 @pytest.mark.parametrize("mode", ["online", "two_pass"])
 def test_prefill_from_a_base_across_chunks_and_query_batches(ctx, mode):
-    """600 queries from row 2,000 of a 2,600-row cache: the queries cross a
-    1,024-token chunk boundary and the 256-query launches of the virtual batch;
-    every query against the C oracle over rows 0 .. base + i."""
+    """600 queries from row 2,000 of a 2,600-row cache, on the kernel that the choice
+    takes (test_gpu_general_kernels runs them as a virtual batch, whose queries cross a
+    1,024-token chunk boundary); every query against the C oracle over rows 0 .. base + i."""
     from insitu_amd.attention import CompressedAttention
     base, n_q = 2000, 600
     T = base + n_q

@@ -70,7 +70,9 @@ def _wire(rng, n, d):
 def test_epoch_wrap_of_each_buffer_in_either_order(ctx):
     """A decode step after a prefill at the prefill buffer's wrap, a prefill after a
     decode at the decode buffer's wrap, and steps on either side of each wrap: every
-    output exact, no chain sent to the serial path."""
+    output exact, no chain sent to the serial path. (The prefill buffer's wrap is reached
+    where the virtual batch is pinned, in test_gpu_general_kernels: unpinned the first
+    prompt leaves the buffer to be allocated, and its count started, by a later one.)"""
     from insitu_amd import _lib
     rng = np.random.default_rng(11)
     d, T0 = 64, 2600

@@ -2,8 +2,10 @@
 insitu_attend_causal (which allocates its scratch) and the C oracle.
 
 Two calls in a row on one device, the second with fewer queries and a different
-base, so the second reuses the static array the first left behind; then a size
-the static array cannot hold is refused before anything runs.
+base: with the virtual batch pinned (test_gpu_general_kernels) the second reuses the
+static array the first left behind, unpinned most of them run on the prefill kernel,
+which needs none. Then a size the static array cannot hold is refused before anything
+runs.
 """
 
 import ctypes
