@@ -924,9 +924,8 @@ static int prefill_kernel_launch(insitu_cache *k, const Geom &gv, int64_t base, 
 static int prefill_launches(insitu_cache *k, const Geom &gv, const PrefillPlan &pl, ChunkScratch &scr,
                             int64_t *len_dev, int64_t base, int64_t n_q, const int32_t *q, int32_t *out,
                             int32_t mode, bool timed = true) {
-    const Geom &g = k->g;
     const bool chunked = mode != INSITU_SERIAL && k->chunked;
-    const int64_t row = (int64_t)g.n_q * g.d;
+    const int64_t row = (int64_t)gv.n_q * gv.d;          // a query of the whole sequence, or of one KV head
     const int64_t qb = chunked ? pl.qb : PREFILL_QB;
     Geom gb = gv;
     for (int64_t i0 = 0; i0 < n_q; i0 += qb) {

@@ -140,6 +140,29 @@ def test_prefill_over_several_launches(ctx, virtual_batch, mode):
 
 
 @pytest.mark.parametrize("mode", ["online", "two_pass"])
+@pytest.mark.parametrize("kb,vb", [(4, 2), (5, 2)])
+def test_one_kv_head_over_several_launches(ctx, virtual_batch, kb, vb, mode):
+    """More queries of one KV head than one launch takes: a later launch's queries and outputs lie at
+    that head's stride, not at the whole sequence's (5-bit keys: the token loop, launched alike)."""
+    from insitu_amd.attention import CompressedAttention
+    base, n, h, f = 5, 1030, 6, Format(key_bits=kb, value_bits=vb)
+    rng = np.random.default_rng(10)
+    k, v = P._random_cache_inputs(rng, base + n)
+    c = P._cache(ctx, base + n, kb=kb, vb=vb)
+    c.append_rotated(k, v)
+    q = rng.integers(-(1 << 22), 1 << 22, size=(n, 4, 64))
+    a = CompressedAttention(c)
+    out, st = (a.attend_online_batch if mode == "online" else a.attend_causal_batch)(q, h, base)
+    host = Cache(8, base + n, f)
+    host.append_rotated(k, v)
+    kv = host.view(h)
+    fn = native.attend_online if mode == "online" else native.attend_two_pass
+    for i in range(n):
+        np.testing.assert_array_equal(out[i], fn(q[i], kv.select(slice(0, base + i + 1)), f)[0], err_msg=f"query {i}")
+    assert st.n_tokens == base + n
+
+
+@pytest.mark.parametrize("mode", ["online", "two_pass"])
 @pytest.mark.parametrize("kb,vb", [(4, 2), (3, 2), (2, 3)])
 def test_prefill_is_the_token_loop(ctx, virtual_batch, kb, vb, mode):
     P.test_prefill_is_the_token_loop(ctx, kb, vb, mode)
