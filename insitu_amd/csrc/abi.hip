@@ -870,12 +870,17 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 // Whether a causal attend runs on the prefill kernel (attend_prefill.hip). Its waves walk their
 // rows' whole contexts, so a grid that does not fill the chip takes a time of its own in the
 // context's length alone; the chunked attend over a virtual batch spreads one query's context over
-// the chip and takes time in proportion to the queries, once they are enough to show over its chain
-// of phases. Fitted to both, measured over 1 to 512 queries of 16 to 4,096 rows, 32 query heads, in
+// the chip and takes time in proportion to the queries and chains, once they are enough to show over
+// its chain of phases. Fitted to both, measured over 1 to 512 queries of 16 to 4,096 rows, 32 query heads, in
 // 4/2- and 3/2-bit codes at d = 64 and 3/3 and 4/2 at d = 128, online and two-pass: the choice takes
 // 0.5 % longer than the better kernel in the mean of them, 1.3 times as long at the worst. E.g. here /
 // there us, d = 64, online: 16 queries of 64 rows 25/27, 256 rows 50/35, 2,048 rows 220/68; 128 of
 // 256 rows 50/83, of 2,048 rows 221/273; d = 128, 3/3 bits: 64 of 512 rows 157/96, 192 263/408 of 1,024.
+// Outside that, 1 to 1,024 queries of 64 to 131,072 rows with 1 to 32 chains of 4 heads (one KV head's
+// attend is one chain), in 4/2 and 3/3 bits: 0.3 % in the mean, 1.18 times at the worst (1.75 when a
+// query cost there what it does with 8 chains: 256 queries of 1,024 rows, one KV head, 139/80).
+// Caches that the chunked attend does not take would go token by token: there 43 us for 64 rows and
+// 0.38 us a row beyond some 1,000 (two-pass 0.58), here 33 and 0.07 (0.085).
 static bool prefill_kernel_takes(const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
     return mode != INSITU_SERIAL && prefill_supported(gv) && base + n_q <= PREFILL_MAX_ROWS;
 }
@@ -887,15 +892,17 @@ static bool prefill_rule(const Geom &gv, bool chunked, int64_t base, int64_t n_q
     // (3-bit codes at d = 128 take most to load and widen; few waves walk a little faster)
     const double walk = (two ? t : near + 0.8 * (t - near)) * (n_q < 32 ? (d64 ? 0.93 : 0.75) : 1.0) *
                         (d64 || gv.kb == 3 ? 1.0 : 0.78);
-    const double work = 1e-5 * t * n * gv.n_q;
+    // the virtual batch's chains of 4 query heads (8 a KV head are two, fewer than 4 are padded)
+    const double chains = (double)gv.n_kv * (gv.G > 4 ? 2 : 1), nc = n * chains / 8.0;
+    const double work = 4e-5 * t * n * chains;
     double here, chain, batch;
     if (d64) {
         here = two ? 11.0 + 0.092 * walk : 18.0 + 0.106 * walk;
-        chain = two ? 22.0 + 0.037 * near + 0.44 * n : 19.0 + 0.042 * near + 0.38 * n;
+        chain = two ? 22.0 + 0.037 * near + 0.44 * nc : 19.0 + 0.042 * near + 0.38 * nc;
         batch = two ? 27.0 + 4.95 * work : 22.0 + 3.0 * work;
     } else {
         here = two ? 15.0 + 0.181 * walk : 25.0 + 0.236 * walk;
-        chain = two ? 28.0 + 0.070 * near + 0.52 * n : 23.0 + 0.092 * near + 0.38 * n;
+        chain = two ? 28.0 + 0.070 * near + 0.52 * nc : 23.0 + 0.092 * near + 0.38 * nc;
         batch = two ? 35.0 + 8.6 * work : 31.0 + 5.6 * work;
     }
     const double there = chain > batch ? chain : batch;

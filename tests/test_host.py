@@ -1,6 +1,7 @@
 """Host-side logic of the product, and the C ABI's surface, without a GPU."""
 
 import ctypes
+import functools
 import os
 import re
 
@@ -315,6 +316,23 @@ def test_causal_attends_past_the_prefill_kernels_rows():
         assert _prefill_rule(lib, 0, 4096, mode) == 1
         assert _prefill_rule(lib, 0, 4096, mode, kb=5) == 0
     assert _prefill_rule(lib, 0, 4096, "serial") == 0
+
+
+@pytest.mark.parametrize("d,kb,vb,rows,n,mode", [(64, 4, 2, 1024, 256, "online"), (64, 4, 2, 1024, 256, "two_pass"),
+                                                 (64, 4, 2, 300, 64, "online"), (128, 3, 3, 1024, 256, "two_pass"),
+                                                 (128, 3, 3, 300, 256, "online")])
+def test_causal_choice_counts_the_chains(d, kb, vb, rows, n, mode):
+    """A query costs the virtual batch less with fewer chains: sizes that all of 8 KV heads run on the
+    prefill kernel and one KV head (a cache's only one, or one of 8) measured faster as a virtual batch;
+    8 query heads a KV head are two chains."""
+    from insitu_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    rule = functools.partial(_prefill_rule, _lib.load(), rows - n, n, mode, d, kb, vb)
+    assert rule(32, 8) == 1 and rule(4, 1) == 0
+    assert rule(32, 4) == 1
+    assert rule(128, 32) == 1
+    assert rule(16, 8) == 1                            # two heads a KV head are padded to four
 
 
 def test_block_chunk_size_follows_capacity():
