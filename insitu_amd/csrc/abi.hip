@@ -714,11 +714,23 @@ static bool use_scan(const insitu_cache *k, int32_t mode) {
 // The fused decode step's own kernel (attend_step.hip), sequential and split mode, wherever
 // it handles the format (d = 64, 4 or 3-bit keys, 2-bit values, 4 query heads per KV head, or 8
 // where the chunked attend sees them as two chains; up to 512 chunks of 1,024 tokens); the test
-// hook can pin the chunked (2) or scan (1) attend. No slower anywhere from 30 to 32,768 tokens and
-// 1 to 64 sequences in the four formats (the kernel's figures).
+// hook can pin the chunked (2) or scan (1) attend. Measured, 3-bit keys, 100 to 131,072 tokens, 1 to 64
+// sequences of 1 or 8 chains, step / chunked step on 1,024-token chunks / on 512, us, flat weights and
+// peaked ones. 4 query heads a KV head: never slower than on 1,024-token chunks (8 KV heads, 16 x
+// 8,192: 120/184/141, 84/107/95); 512 ones, which a cache takes for flat weights, gain 1 to 11 % there and
+// lose 3 to 12 % on peaked ones between 1,000 and 16,384 tokens of a few sequences (1,000: 31/49/35,
+// 26/29/24). 8 query heads (the chunked step: a write launch, and two attend workgroups a CU): 0.64 to
+// 0.92 of either on flat weights and on peaked ones of up to 256 chunks in all, a workgroup a CU
+// (4 KV heads, 8,192: 34/69/47, 27/36/32); beyond, peaked weights take longer (16 x 8,192: 120/147/160,
+// 86/66/80; 16 x 32,768: 398/500/554, 244/158/217), so that there only the caches that expect flat ones,
+// those of 512-token chunks, take it.
 static bool use_step_kernel(const insitu_cache *k, int32_t mode) {
     if ((mode != INSITU_SEQUENTIAL && mode != INSITU_SPLIT) || !k->step) return false;
-    return k->path != 1 && k->path != 2;
+    if (k->path == 1 || k->path == 2) return false;
+    if (k->path == 3 || !k->vsplit || k->api->tokens == 512) return true;
+    int64_t chunks = 0;
+    for (int64_t n : k->len_host) chunks += step_max_chunks(n + 1);
+    return chunks * k->g.n_kv * 2 <= 256;
 }
 
 // The split attend: pinned (4), or automatically in two-pass mode, where the chunked attend scores

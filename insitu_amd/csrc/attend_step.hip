@@ -7,8 +7,8 @@
 // Bounds: the chain of dependent phases up to some 8,192 tokens, then the fp64 scores and the walk.
 // Steps with 3-bit keys, 2,047 tokens, before (the chunked attend: with 8 query heads a write launch
 // and an attend launch, 2 chains a KV head either way) and here, flat and peaked weights: 4 heads
-// 35 -> 33 and 22 -> 21 us, x 64 sequences 203 -> 147 and 156 -> 96; 8 heads (4 KV heads) 47 -> 33 and
-// 28 -> 21, x 64 sequences 179 -> 147 and 103 -> 96.
+// 35 -> 33 and 22 -> 21 us; 8 heads (4 KV heads) 47 -> 33 and 28 -> 21. Over more sizes and sequences,
+// and where the chunked step stays the faster one: use_step_kernel (abi.hip).
 //
 // The arithmetic is the chunked attend's (attend_chunked.hip): a chunk knows the
 // running maximum before it (M_in, by a decoupled look-back over its predecessors'

@@ -84,3 +84,34 @@ def test_the_look_back_giving_up(ctx, kb, G):
 @pytest.mark.parametrize("kb,G", FORMATS)
 def test_range_errors_are_counted_once(ctx, kb, G):
     assert _run(ctx, kb, G, [70], 1, 1 << 13, outlier=True)["range_errors"] > 0
+
+
+@pytest.mark.parametrize("chunk_tokens", [512, 1024])
+@pytest.mark.parametrize("longer", [0, 1])
+def test_either_side_of_the_choice(ctx, longer, chunk_tokens):
+    """8 query heads a KV head: 256 chunks in all (64 sequences, 4 chains) and 260, where caches of
+    1,024-token chunks go back to the chunked step; the automatic choice against both kernels."""
+    import torch
+    from insitu_amd import QuantConfig, _lib
+    from insitu_amd.cache import CompressedCache
+    from insitu_amd.runtime import ptr
+    batch, n, G = 64, 1023, 8
+    rng = np.random.default_rng(longer)
+    draw = lambda s, *shape: ctx.to_device(np.rint(rng.standard_normal(shape) * s).astype(np.int64), torch.int32)
+    k, v = draw(65536, n + 1, N_KV, D), draw(65536, n + 1, N_KV, D)
+    q, kk, vv = draw(16384, batch, N_KV * G, D), draw(65536, batch, N_KV, D), draw(65536, batch, N_KV, D)
+    res = []
+    for pin in ("auto", "step", "chunked"):
+        c = CompressedCache(N_KV, D, n + 3, QuantConfig(key_bits=3, value_bits=2), batch=batch, n_q_heads=N_KV * G,
+                            chunk_tokens=chunk_tokens, ctx=ctx)
+        for b in range(batch):
+            m = n + (longer if b == 5 else 0)
+            c.append_rotated(k[:m], v[:m], seq=b)
+        c.pin_kernel(pin)
+        out, st = torch.empty_like(q), _lib.Stats()
+        _lib.check(ctx.lib.insitu_step(c.handle, ptr(q), ptr(kk), ptr(vv), ptr(out), _lib.SEQUENTIAL, st))
+        res.append((out, [getattr(st, f) for f, _ in st._fields_], [c.read_rows(1, n, 1, seq=b) for b in (0, 5, 63)]))
+        assert c.lengths() == [n + 1 + (longer if b == 5 else 0) for b in range(batch)]
+    for r in res[1:]:
+        assert torch.equal(r[0], res[0][0]) and r[1] == res[0][1]
+        np.testing.assert_array_equal(r[2], res[0][2])
