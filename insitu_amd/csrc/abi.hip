@@ -883,14 +883,15 @@ PrefillPlan prefill_plan(const ChunkedApi &api, const Geom &gv, int64_t base, in
 // rows' whole contexts, so a grid that does not fill the chip takes a time of its own in the
 // context's length alone; the chunked attend over a virtual batch spreads one query's context over
 // the chip and takes time in proportion to the queries and chains, once they are enough to show over
-// its chain of phases. Fitted to both, measured over 1 to 512 queries of 16 to 4,096 rows, 32 query heads, in
-// 4/2- and 3/2-bit codes at d = 64 and 3/3 and 4/2 at d = 128, online and two-pass: the choice takes
-// 0.5 % longer than the better kernel in the mean of them, 1.3 times as long at the worst. E.g. here /
-// there us, d = 64, online: 16 queries of 64 rows 25/27, 256 rows 50/35, 2,048 rows 220/68; 128 of
-// 256 rows 50/83, of 2,048 rows 221/273; d = 128, 3/3 bits: 64 of 512 rows 157/96, 192 263/408 of 1,024.
-// Outside that, 1 to 1,024 queries of 64 to 131,072 rows with 1 to 32 chains of 4 heads (one KV head's
-// attend is one chain), in 4/2 and 3/3 bits: 0.3 % in the mean, 1.18 times at the worst (1.75 when a
-// query cost there what it does with 8 chains: 256 queries of 1,024 rows, one KV head, 139/80).
+// its chain of phases. Fitted to both, measured over 1 to 512 queries of 16 to 4,096 rows, 32 query heads,
+// in 4/2- and 3/2-bit codes at d = 64 and 3/3 and 4/2 at d = 128, online and two-pass. E.g. here / there
+// us, calls waited for, online: d = 64, 4/2 bits, 16 queries of 64 rows 35/39, of 300 65/50, of 2,048
+// 237/82; 128 of 300 rows 69/100, of 2,048 236/306; d = 128, 3/3 bits, 64 of 600 rows 188/108, 256 of 1,024
+// 282/451.
+// Over 1,508 calls of 1 to 1,024 queries of 16 to 131,072 rows, 1 to 32 chains of 4 heads (one KV head's
+// attend is one chain) and ten formats with 2- to 4-bit keys and 1- to 3-bit values the choice takes 0.4 %
+// longer than the better kernel in the mean, 1.24 times as long at the worst (64 queries of 150 rows, 3/3 bits,
+// d = 128: 85/68).
 // Caches that the chunked attend does not take would go token by token: there 43 us for 64 rows and
 // 0.38 us a row beyond some 1,000 (two-pass 0.58), here 33 and 0.07 (0.085).
 static bool prefill_kernel_takes(const Geom &gv, int64_t base, int64_t n_q, int32_t mode) {
@@ -901,9 +902,9 @@ static bool prefill_rule(const Geom &gv, bool chunked, int64_t base, int64_t n_q
     if (!chunked) return true;              // else token by token
     const bool two = mode == INSITU_TWO_PASS, d64 = gv.d == 64;
     const double t = (double)(base + n_q), near = t < 1024.0 ? t : 1024.0, n = (double)n_q;
-    // (3-bit codes at d = 128 take most to load and widen; few waves walk a little faster)
+    // (3-bit values have twice the terms and one-hot codes; few waves walk a little faster)
     const double walk = (two ? t : near + 0.8 * (t - near)) * (n_q < 32 ? (d64 ? 0.93 : 0.75) : 1.0) *
-                        (d64 || gv.kb == 3 ? 1.0 : 0.78);
+                        (gv.vb > 2 ? (d64 ? 1.1 : 1.0) : (d64 ? 1.0 : 0.78));
     // the virtual batch's chains of 4 query heads (8 a KV head are two, fewer than 4 are padded)
     const double chains = (double)gv.n_kv * (gv.G > 4 ? 2 : 1), nc = n * chains / 8.0;
     const double work = 4e-5 * t * n * chains;

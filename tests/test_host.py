@@ -335,6 +335,18 @@ def test_causal_choice_counts_the_chains(d, kb, vb, rows, n, mode):
     assert rule(16, 8) == 1                            # two heads a KV head are padded to four
 
 
+@pytest.mark.parametrize("d,kb,rows,n", [(128, 4, 150, 48), (64, 2, 300, 48), (64, 3, 300, 48)])
+def test_causal_choice_counts_the_value_bits(d, kb, rows, n):
+    """3-bit values take the prefill kernel longer, whatever the keys: sizes that 2-bit values run there
+    and 3-bit ones measured faster as a virtual batch."""
+    from insitu_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.load()
+    assert _prefill_rule(lib, rows - n, n, "online", d, kb, 2) == 1
+    assert _prefill_rule(lib, rows - n, n, "online", d, kb, 3) == 0
+
+
 def test_block_chunk_size_follows_capacity():
     """A block's cache takes 512-token chunks only while the chunked attend's chunk limit
     holds them; past 262,144 tokens it keeps 1,024-token chunks (and the chunked path)."""
