@@ -468,20 +468,34 @@ bool gemv_fits(int64_t n, int32_t in_f) {
     return n <= GEMV_N && in_f % 8 == 0;
 }
 
+// 64 x 64 tiles where they give every CU a workgroup, else 32 x 32 (2,048 -> 2,048, 512 tokens: 20.1 us,
+// 23.6 in 32 x 32; 2,048 -> 3,072, 128 tokens in 32 x 32: 11.9)
+bool gemm_big(int64_t n, int32_t out_f) { return ((n + 63) / 64) * (((int64_t)out_f + 63) / 64) >= 256; }
+
 // The prompt's projections on gemm_f16_kernel: 16-byte loads, so channels in eights and aligned rows;
-// up to 2^31 multiply-adds. rocBLAS takes 26 to 28 us a call whatever the size up to there (its call
-// and the cast's launch), and its tiles are the faster ones beyond. Here / there, us, 2,048 -> 3,072
-// from fp32: 5 to 64 tokens 9/27, 256 16/27, 333 24/27, 700 39/27; 2,048 -> 2,048 from Q16: 64 tokens
-// 13/27, 512 20/26, 700 28/26; 4,096 -> 6,144: 5 tokens 19/27, 64 21/27, 128 27/27, 256 43/40.
-bool gemm_fits(const void *w, const void *x, int64_t n, int32_t out_f, int32_t in_f) {
-    return in_f % 8 == 0 && (((uintptr_t)w | (uintptr_t)x) & 15) == 0 && n <= (int64_t(1) << 31) / out_f / in_f;
+// where it takes no longer than a rocBLAS call, which is 21 to 28 us by the host whatever the size (its
+// call and the cast's launch) until the product itself takes longer, and then has the faster tiles. Here
+// a workgroup is a chain of 128-channel steps, more workgroups on a CU slow each other, and the weights
+// come in at 3.7 TB/s: up to 25 us within 4 us of what 13 shapes of 512 to 16,384 channels and outputs and 5 to
+// 2,048 tokens measured. cast: a Q16 output is cast by a launch of its own either way (2 us more here, where
+// the host does not hide it). Here / there us on a box of 21, from fp32: 2,048 -> 3,072, 5 to 64 tokens 9/21,
+// 256 16/21, 333 25/21; 4,096 -> 6,144, 5 tokens 19/21, 64 22/21; 1,024 -> 1,536, 700 16/21; 8,192 -> 10,240,
+// 5 tokens 41/31; 16,384 -> 2,048, 5 tokens 58/23; from Q16, 2,048 -> 2,048, 512 tokens 20/23.
+bool gemm_fits(const void *w, const void *x, int64_t n, int32_t out_f, int32_t in_f, bool cast) {
+    if (in_f % 8 != 0 || (((uintptr_t)w | (uintptr_t)x) & 15) != 0 || n > (int64_t(1) << 31) / out_f / in_f) return false;
+    const bool big = gemm_big(n, out_f);
+    const int64_t bt = big ? 64 : 32, wgs = ((n + bt - 1) / bt) * (((int64_t)out_f + bt - 1) / bt);
+    const double steps = (in_f + 127) / 128, deep = (double)((wgs + 255) / 256);       // workgroups a CU
+    const double rounds = big ? (double)((wgs + 511) / 512) : 1.0;                     // (two of 64 x 64 fit)
+    const double chain = big ? rounds * (5.0 + steps * (0.5 + 0.4 * (deep < 2.0 ? deep : 2.0)))
+                             : 1.5 + steps * (0.23 + 0.225 * deep);
+    const double weights = 2.5 + 2.0 * out_f * in_f / 3.7e6;
+    return (chain > weights ? chain : weights) + (cast ? 2.0 : 0.0) <= 21.5;
 }
 
 template <typename XT>
 int gemm(insitu_ctx *c, const uint16_t *w, int32_t out_f, int32_t in_f, const XT *x, int64_t n, const float *bias, float *y) {
-    // 64 x 64 tiles where they give every CU a workgroup, else 32 x 32 (2,048 -> 2,048, 512 tokens: 20.1 us,
-    // 23.6 in 32 x 32; 2,048 -> 3,072, 128 tokens in 32 x 32: 11.9)
-    const bool big = ((n + 63) / 64) * (((int64_t)out_f + 63) / 64) >= 256;
+    const bool big = gemm_big(n, out_f);
     const int bt = big ? 64 : 32;
     const int64_t toks = (n + bt - 1) / bt, outs = ((int64_t)out_f + bt - 1) / bt, grid = (outs + 7) / 8 * 8 * toks;
     if (big)
@@ -557,7 +571,7 @@ int insitu_project(insitu_ctx *c, const uint16_t *w, int32_t out_f, int32_t in_f
     if (n == 0) return INSITU_OK;
     HIP_TRY(hipSetDevice(ctx_device(c)), "hipSetDevice");
     if (gemv_fits(n, in_f)) return gemv<false>(c, w, out_f, in_f, x, n, 0.0, bias, y);
-    if (gemm_fits(w, x, n, out_f, in_f)) return gemm(c, w, out_f, in_f, x, n, bias, y);
+    if (gemm_fits(w, x, n, out_f, in_f, false)) return gemm(c, w, out_f, in_f, x, n, bias, y);
     int rc = ensure_x16(c, (size_t)n * in_f);
     if (rc) return rc;
     Blas &b = blas_of(c);
@@ -646,7 +660,7 @@ int insitu_output_projection(insitu_ctx *c, const int32_t *out, int64_t n, int32
         hipLaunchKernelGGL(fixed_to_f16_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, ctx_stream(c), out,
                            b.x16, nx, std::ldexp(1.0, -frac));
     HIP_TRY(hipGetLastError(), "fixed to fp16");
-    if (gemm_fits(wo, b.x16, n, hidden, width)) return gemm(c, wo, hidden, width, b.x16, n, bias, y);
+    if (gemm_fits(wo, b.x16, n, hidden, width, true)) return gemm(c, wo, hidden, width, b.x16, n, bias, y);
     rc = gemm_f16(c, wo, hidden, width, b.x16, n, y);
     if (rc) return rc;
     if (bias) {

@@ -47,3 +47,9 @@ def test_projection_tiles(ctx, n, out_f, in_f, shift, biased):
         od = placed(o)
         _lib.check(ctx.lib.insitu_output_projection(ctx.handle, ptr(od), n, in_f, frac, ptr(wd), out_f, bias, ptr(y)))
         _check(y.cpu().numpy().astype(np.float64), w, (o.astype(np.float64) / 2.0**frac).astype(np.float16), b)
+
+
+@pytest.mark.parametrize("biased", [False, True])
+def test_large_tiles(ctx, biased):
+    """64 x 64 tiles (264 workgroups) with remainders of tokens, outputs and channels."""
+    test_projection_tiles(ctx, 700, 1500, 1000, 0, biased)
