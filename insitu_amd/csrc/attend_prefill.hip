@@ -8,14 +8,15 @@
 // waited for and nothing is published or replayed. A workgroup's waves share one KV head's
 // tokens, which they expand together into matrix operands in LDS, double-buffered.
 //
-// Scores. dot = sum_ch q[ch] * c[code_ch] is exact: q in four balanced signed bytes, the key
-// centroids in three, v_mfma_i32_16x16x64_i8 over the channels for every pair of digits, the
-// products of equal weight in one int32 accumulator (at most 4 * 2 * 2^20 < 2^31 there). The
-// fourth byte of q is skipped when every value of the wave's rows fits three. The six sums
-// combine in fp64 (exact: |dot| <= ||q||_1 max|c| < 2^51, else the row goes to the serial
-// path). dot * k_norm / 2^24 is exact in fp64 below 2^53; one bound a stage proves it, else
-// the products are looked at, and if one is too large the workgroup starts again with int64
-// scores (WIDE), which cover everything the reference computes.
+// Scores. dot = sum_ch q[ch] * c[code_ch] exactly: q and the key centroids in three balanced signed
+// bytes each, v_mfma_i32_16x16x64_i8 over the channels for every pair of digits, the products of
+// equal weight in one int32 accumulator that carries into the next lower weight's: dot = 2^16 H + L.
+// floor(dot k_norm / 2^24) is then int64 arithmetic, and the scores int32. Where that does not do (a
+// value of q that needs its fourth byte, ||q||_1 max|c| from 2^46 on, a product past 2^55, which one
+// bound a stage excludes or else the products are looked at, or a value term past three digits) the
+// workgroup starts again with four digits and int64 scores (WIDE), which cover everything the
+// reference computes: an int64 shifted right by 24 never reaches the 48-bit clamp, so that no score
+// of this kernel overflows. A row with ||q||_1 max|c| from 2^51 on goes to the serial path.
 //
 // The matrix product's result has lane = (row, 4 tokens): the running maximum, the exp LUT and
 // the terms floor(v_norm p c_v / 2^23) for every value code are computed there, and the terms'
@@ -124,7 +125,7 @@ struct Lds {
     alignas(16) uint32_t dig[3][4];                    // 16 centroids' digits, a byte each
     uint16_t lut[LUT_N + 7];
     int rerun;
-    unsigned long long events, sovf, rerr, fallbacks, mabs, macc;
+    unsigned long long events, rerr, fallbacks, mabs, macc;
 };
 
 // A workgroup's walk over its tokens, and its rows' outputs. Narrow scores: returns true when
@@ -156,7 +157,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     if (tid == 0) {
         // (not in the wide walk: a wave of this workgroup may still be about to read it there)
         if constexpr (!WIDE) S.rerun = 0;
-        S.events = S.sovf = S.rerr = S.fallbacks = S.mabs = S.macc = 0;
+        S.events = S.rerr = S.fallbacks = S.mabs = S.macc = 0;
     }
     const int kb = g.kb, vb = g.vb;
     if (tid < 256) {
@@ -350,7 +351,7 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     v4i acc[C::CT];                                    // lane = (row, 4 channels of each tile)
     uint32_t lp = 0;                                   // this lane's part of the denominator since the last event or fold
     uint64_t l64 = 0;                                  // the row's denominator up to there
-    uint32_t n_events = 0, n_sovf = 0;
+    uint32_t n_events = 0;
     float bsum = 0.0f;                                 // bound of |acc| over the wave's rows
 #pragma unroll
     for (int c = 0; c < C::CT; ++c) acc[c] = v4i{0, 0, 0, 0};
@@ -493,14 +494,6 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             }
         }
         const int32_t tg = t0 + grp * 4;               // this lane's first token
-        if constexpr (WIDE) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const bool o = s[i] < (SC)SCORE_LO || s[i] > (SC)SCORE_HI;
-                if (P != FIXEDMAX && o && tg + i < limit) ++n_sovf;
-                if (o) s[i] = s[i] < 0 ? (SC)SCORE_LO : (SC)SCORE_HI;
-            }
-        }
         if (diag) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -764,11 +757,10 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
             if (mine) *(u128 *)(out + at + c * 16 + grp * 4) = u128{o[0], o[1], o[2], o[3]};
         }
         const int64_t mp = (int64_t)m < 0 ? -(int64_t)m : (int64_t)m, mn = -(int64_t)smin;
-        const int64_t ev = wave_sum_i64(mine ? n_events : 0), ov = wave_sum_i64(mine ? n_sovf : 0);
+        const int64_t ev = wave_sum_i64(mine ? n_events : 0);
         const int64_t ma = wave_max_i64(mine ? (mp > mn ? mp : mn) : 0), mc = wave_max_i64(mine ? macc : 0);
         if (lane == 0) {
             if (ev) atomicAdd(&S.events, (unsigned long long)ev);
-            if (ov) atomicAdd(&S.sovf, (unsigned long long)ov);
             atomicMax(&S.mabs, (unsigned long long)ma);
             atomicMax(&S.macc, (unsigned long long)mc);
         }
@@ -789,7 +781,6 @@ __device__ __forceinline__ bool prefill_rows(const Geom &g, const Tables *__rest
     // it is one as far as this workgroup can see
     if (tid == 0) {
         if (S.events) atomicAdd(&st->rescale_events, S.events);
-        if (S.sovf) atomicAdd(&st->score_overflows, S.sovf);
         if (S.rerr) atomicAdd(&st->range_errors, S.rerr);
         if (S.fallbacks) atomicAdd(&st->serial_fallbacks, S.fallbacks);
         if (S.mabs > st->max_abs_score) atomicMax(&st->max_abs_score, S.mabs);
