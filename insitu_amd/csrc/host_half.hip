@@ -473,14 +473,17 @@ bool gemv_fits(int64_t n, int32_t in_f) {
 bool gemm_big(int64_t n, int32_t out_f) { return ((n + 63) / 64) * (((int64_t)out_f + 63) / 64) >= 256; }
 
 // The prompt's projections on gemm_f16_kernel: 16-byte loads, so channels in eights and aligned rows;
-// where it takes no longer than a rocBLAS call, which is 21 to 28 us by the host whatever the size (its
-// call and the cast's launch) until the product itself takes longer, and then has the faster tiles. Here
-// a workgroup is a chain of 128-channel steps, more workgroups on a CU slow each other, and the weights
-// come in at 3.7 TB/s: up to 25 us within 4 us of what 13 shapes of 512 to 16,384 channels and outputs and 5 to
-// 2,048 tokens measured. cast: a Q16 output is cast by a launch of its own either way (2 us more here, where
-// the host does not hide it). Here / there us on a box of 21, from fp32: 2,048 -> 3,072, 5 to 64 tokens 9/21,
-// 256 16/21, 333 25/21; 4,096 -> 6,144, 5 tokens 19/21, 64 22/21; 1,024 -> 1,536, 700 16/21; 8,192 -> 10,240,
-// 5 tokens 41/31; 16,384 -> 2,048, 5 tokens 58/23; from Q16, 2,048 -> 2,048, 512 tokens 20/23.
+// where it takes no longer than a rocBLAS call and the cast's launch. Those take 21 to 28 us (by the
+// host) a call among others and 39 to 42 when the GPU is waited for, whatever the size, until the
+// product itself takes longer, and then has the faster tiles. Here a workgroup is a chain of
+// 128-channel steps, more workgroups on a CU slow each other, and the weights come in at 3.7 TB/s: up to
+// 25 us within 4 us of what 13 shapes of 512 to 16,384 channels and outputs and 5 to 2,048 tokens
+// measured. cast: a Q16 output is cast by a launch of its own either way (2 us more here, where the host
+// does not hide it). The line lies between the two: at it a call among others takes up to 1.1 times as
+// long as there on the fastest host, and one waited for 0.85. Here / there us among others, and waited for:
+// 2,048 -> 3,072, 64 tokens 9/24, 333 25/24, 35/41; 4,096 -> 6,144, 64 tokens 23/24, 34/42; 5,120 -> 7,168, 5
+// tokens 23/24, 33/41; 8,192 -> 10,240, 5 tokens 41/32, 51/54; 16,384 -> 2,048, 5 tokens 58/24, 68/42; from
+// Q16, 2,048 -> 2,048, 512 tokens 20/24.
 bool gemm_fits(const void *w, const void *x, int64_t n, int32_t out_f, int32_t in_f, bool cast) {
     if (in_f % 8 != 0 || (((uintptr_t)w | (uintptr_t)x) & 15) != 0 || n > (int64_t(1) << 31) / out_f / in_f) return false;
     const bool big = gemm_big(n, out_f);
@@ -490,7 +493,7 @@ bool gemm_fits(const void *w, const void *x, int64_t n, int32_t out_f, int32_t i
     const double chain = big ? rounds * (5.0 + steps * (0.5 + 0.4 * (deep < 2.0 ? deep : 2.0)))
                              : 1.5 + steps * (0.23 + 0.225 * deep);
     const double weights = 2.5 + 2.0 * out_f * in_f / 3.7e6;
-    return (chain > weights ? chain : weights) + (cast ? 2.0 : 0.0) <= 21.5;
+    return (chain > weights ? chain : weights) + (cast ? 2.0 : 0.0) <= 26.5;
 }
 
 template <typename XT>
