@@ -374,8 +374,8 @@ __device__ __forceinline__ void score_keys(const uint32_t (&w)[TPT][KF<D, KB>::K
 // lanes that own the tokens. A centroid then costs a byte permute for each of its 3 digits and 4
 // channels, where the fp64 score reads 8 bytes of LDS and issues 4 FMAs a (token, channel): a CU's LDS
 // and its FMAs bounded the attend of large batches. 16 sequences of 131,072 rows, d = 128, 3-bit keys
-// and values: 739 us a call (810 with the fp64 score; 2.3 TB/s); 64 of 1,024 to 8,192 rows, d = 64,
-// 4/2 bits: 111.3 (112.5: its chunks are few a CU, and the chain of phases behind the score bounds it).
+// and values: 732 us a call (812 with the fp64 score; 2.3 TB/s); 64 of 1,024 to 8,192 rows, d = 64,
+// 4/2 bits: 110.8 (112.3: its chunks are few a CU, and the chain of phases behind the score bounds it).
 template <int D, int KB>
 __device__ __forceinline__ void score_mfma(const uint32_t (&w)[TPT][KF<D, KB>::KWORDS + 1],
                                            const uint32_t (&normw)[TPT], const int32_t *qb,
@@ -592,6 +592,9 @@ __global__ void __launch_bounds__(CT) chunk_max_kernel(Geom g, const Tables *__r
 // token more: every workgroup rotates its group's wire query rows itself, and
 // the workgroup of the chunk holding the new token rotates, encodes and packs
 // its key/value row, stores it into the planes and scores it from LDS.
+// At d = 128 the bound of 128 registers keeps two workgroups on a CU; 4-bit keys spill 11 of them for it
+// (4/2-bit codes within 2 % of the fp64 scores' time at 1,000 to 65,536 rows, 16 x 131,072 rows in 3/3-bit
+// codes 732 us, 812 before).
 template <int D, int KB, bool SEQ, bool QS, bool STEP>
 __global__ void __launch_bounds__(CT, SEQ && D > 64 ? 4 : 2) chunk_kernel(Geom g, const Tables *__restrict__ tabs,
                                                    const int32_t *__restrict__ q,

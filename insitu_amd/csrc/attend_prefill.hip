@@ -34,14 +34,17 @@
 // wave proves it, refreshed from the accumulators when it gets large; a row where it cannot be
 // proven is recomputed on the serial path (serial_head.h), as is one whose scores are not exact.
 //
-// What bounds it: VALU issue (about 180 instructions a 16 x 16 tile without an event, 5 cycles
-// each at 2 waves a SIMD and 7 to 11 for a wave alone; the products take a fifth of the time), and
-// the tiles with events (about half of a 4,096-token prompt's, twice the instructions). One
-// accumulator instead of one a digit costs two VALU instructions a register and tile and frees 32
-// registers at d = 64 (64 at 128), which there is what keeps the walk free of spills.
-// Measured (the attend, Llama-3.2-1B shape, queries scaled as a model's): 4,096 tokens 865 us
-// (8,632 on the virtual batch of decode attends before), unscaled 807 (3,560); 333 tokens behind
-// 2,000 243 us (797); 1,000 tokens at d = 128, 3b/3b, two-pass 210 us (1,923), online 265 (1,130).
+// What bounds it (SQ counters): VALU issue. A 4,096-token prompt takes a wave
+// some 330 VALU and 25 matrix instructions a 16 x 16 tile, its share of the staging and its events
+// included; they fill 62 % and 19 % of the SIMDs' cycles. 28 % of its tiles hold events (a count of
+// random rows drawn as the benchmark's). A short prompt, two waves a SIMD or one, is bound by the
+// longest walk's own latency: 0.1 us a row at d = 64, 0.1 a row and pass at d = 128. One accumulator
+// instead of one a digit costs two VALU instructions a register and tile and frees 32 registers at
+// d = 64 (64 at 128); the walk still spills some: 46 registers online and 42 two-pass at the 168 of three
+// workgroups a CU, 26 to 62 at d = 128's 256.
+// Measured (the kernel, Llama-3.2-1B shape, queries scaled as a model's): 4,096 tokens 883 us (the
+// call 8,632 on the virtual batch of decode attends before); 333 tokens behind 2,000 219 us (797);
+// 1,000 tokens at d = 128, 3b/3b, two-pass 201 us (1,923).
 #include <type_traits>
 
 #include "digits.h"

@@ -18,7 +18,8 @@ __device__ __forceinline__ v4i mma(v4i rows, v4i cols, v4i c) {
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);         // selector bytes 0-3: lo, 4-7: hi, 12: zero
 }
-// The balanced digits 0 to 2 of x as bytes 0 to 2, and digit 3 as byte 3 (|x| < 2^31 - 2^23).
+// The balanced digits 0 to 2 of x as bytes 0 to 2, and digit 3 as byte 3 (x at most 2^31 - 1 - 0x808080:
+// from there on x + 0x808080 leaves int32).
 __device__ __forceinline__ uint32_t balanced(int32_t x) { return ((uint32_t)x + 0x808080u) ^ 0x808080u; }
 
 // The digits of 16 key centroids, dg[i][j] holding digit i of centroids 4 j .. 4 j + 3.

@@ -296,8 +296,9 @@ struct ChunkedApi {
                          const int64_t *, ChunkScratch &, uint32_t, int64_t, int64_t, int, bool,
                          const StepIn *, LaunchEv, DevStats *, int64_t, int64_t);
 };
-// The fused decode step's own kernel (attend_step.hip): sequential mode at d = 64, 4 query
-// heads per KV head, 4-bit keys and 2-bit values, 1,024-token chunks of 16 waves. It lays the
+// The fused decode step's own kernel (attend_step.hip): sequential mode at d = 64, 2-bit values,
+// 4-bit keys and 4 query heads per KV head, or 3-bit keys and 4 or (as two chains) 8;
+// 1,024-token chunks of 16 waves. It lays the
 // chunk scratch out its own way (scratch_layout clears the front when the layout changes).
 // The scratch layouts' invariants, for a host-side test (insitu_debug_scratch_layout):
 // f[0] chunks the layout is for, f[1] run slots per head (pool), f[2] slots per chunk after
@@ -320,9 +321,8 @@ hipError_t launch_step_write(hipStream_t s, const Geom &g, const Tables *t, cons
                              const int32_t *kw, const int32_t *vw, int rounds,
                              const uint64_t (*signs)[2], int32_t *qr, double *qd, int32_t *qok,
                              const int64_t *len_in, int64_t *len_out, DevStats *st);
-// The two-pass attend in two launches (attend_split.hip): one query a sequence, or with step the whole decode step
-// (len the lengths before it); longest: the longest sequence, the new token
-// included.
+// The two-pass attend in two launches (attend_split.hip): one query a sequence, or with step the whole
+// decode step (len the lengths before it); longest: the longest sequence, the new token included.
 bool split_supported(const Geom &g, const Tables &host_tabs, int64_t capacity);
 size_t split_scratch_bytes(const Geom &g, int64_t capacity);
 hipError_t launch_attend_split(hipStream_t s, const Geom &g, const Tables *t, const int32_t *q, int32_t *out,

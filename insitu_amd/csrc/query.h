@@ -1,14 +1,14 @@
 // The query side of the chunked attend.
 //
-// Each KV group's GF rotated query rows are staged once per call as fp64, in
-// the layout [chain][channel][head] (chain = sequence * n_kv + KV head), by the
-// kernel that produces them: the rotation of the fused decode step, or the
-// query-prep kernel in front of a standalone attend. Every workgroup of the
-// chain then reads them through scalar loads and uses them as the scalar
-// operand of its score FMAs, so the scoring loop reads only the key centroids
-// from LDS. A per-chain flag records whether every score of the group stays
-// an exact fp64 integer (attention.py:333-359 computes them in int64):
-// |dot| <= ||q||_1 * max|c| < 2^51.
+// Where a launch goes before the attend (two-pass mode; d = 128), each KV group's GF rotated query
+// rows are staged once per call as fp64, in the layout [chain][channel][head] (chain = sequence * n_kv
+// + KV head), by the kernel that produces them: the rotation of the fused decode step, the query-prep
+// kernel in front of a standalone attend, or chunk_max_kernel. chunk_max_kernel's workgroups read
+// staged rows through scalar loads as the scalar operand of their score FMAs; chunk_kernel's read a
+// value a thread and turn it into the digits of its matrix-core scores (digits.h). Elsewhere a
+// workgroup stages its own rows in LDS. A per-chain flag records whether every score of the group is
+// exact that way (attention.py:333-359 computes them in int64): |dot| <= ||q||_1 * max|c| < 2^51, and
+// every value has balanced digits.
 #pragma once
 
 #include "insitu_internal.h"
