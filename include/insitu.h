@@ -291,12 +291,12 @@ enum {
                                         up at once, sending every chain with a predecessor to the
                                         exact serial path                                       */
     INSITU_DEBUG_PATH = 4,           /* the kernel of a sequential-mode attend: 0 automatic (the
-                                        decode step on its own kernel where it handles the cache,
-                                        the chunked attend where it handles the cache, the scan
-                                        attend elsewhere), 1 the scan attend, 2 the chunked attend
-                                        (the decode step too), 3 the decode step's own kernel,
-                                        4 two-pass mode's split attend
-                                        (any other mode automatic);
+                                        decode step on its own kernel where it handles the cache
+                                        and is the faster one, the chunked attend where it handles
+                                        the cache, the scan attend elsewhere), 1 the scan attend, 2
+                                        the chunked attend (the decode step too), 3 the decode
+                                        step's own kernel, 4 two-pass mode's split attend (any
+                                        other mode automatic);
                                         INSITU_EINVAL if the kernel does not handle the cache   */
     INSITU_DEBUG_APPEND = 5,         /* the append's kernel: 0 automatic (lane = row for more
                                         than 4,096 rows where it handles the format: d = 64, 4/2-

@@ -381,10 +381,11 @@ class CompressedCache(KVCache):
 
     def pin_kernel(self, path: str) -> None:
         """Test hook: the kernel of sequential-mode attends on this cache, "auto" (the
-        decode step's own kernel for insitu_step where it handles the format, the chunked
-        attend where it handles the format and capacity, the scan attend elsewhere),
-        "scan", "chunked" (the decode step too), "step" (the decode step's own kernel) or
-        "split" (two-pass mode's two launches; other modes automatic). Raises if that kernel does not handle the cache."""
+        decode step's own kernel for insitu_step where it handles the format and is the
+        faster one, the chunked attend where it handles the format and capacity, the scan
+        attend elsewhere), "scan", "chunked" (the decode step too), "step" (the decode step's
+        own kernel) or "split" (two-pass mode's two launches; other modes automatic). Raises
+        if that kernel does not handle the cache."""
         code = {"auto": _lib.PATH_AUTO, "scan": _lib.PATH_SCAN, "chunked": _lib.PATH_CHUNKED,
                 "step": _lib.PATH_STEP, "split": _lib.PATH_SPLIT}[path]
         _lib.check(self.ctx.lib.insitu_cache_debug(self.handle, _lib.DEBUG_PATH, code))
