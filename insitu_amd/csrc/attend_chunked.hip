@@ -427,8 +427,10 @@ __device__ __forceinline__ void score_mfma(const uint32_t (&w)[TPT][KF<D, KB>::K
             }
         }
         wave_sync();
-#pragma unroll 2
-        for (int tile = 0; tile < NT / 16; ++tile) {       // (by 4 it takes 3 to 10 registers more than there are)
+        // (by 4 it takes 3 to 10 registers more than there are; 4-bit keys at d = 128 by 2 already 11: attends of
+        // their formats took up to 1.05 of the fp64 scores' time that way, 1.02 one by one)
+#pragma unroll (D == 128 && KB == 4 ? 1 : 2)
+        for (int tile = 0; tile < NT / 16; ++tile) {
             // channels [grp D / 4, (grp + 1) D / 4) of token `col` of the tile
             const uint32_t *row = kbuf + (16 * tile + col) * KW;
             uint64_t code[CPL];
@@ -592,7 +594,7 @@ __global__ void __launch_bounds__(CT) chunk_max_kernel(Geom g, const Tables *__r
 // token more: every workgroup rotates its group's wire query rows itself, and
 // the workgroup of the chunk holding the new token rotates, encodes and packs
 // its key/value row, stores it into the planes and scores it from LDS.
-// At d = 128 the bound of 128 registers keeps two workgroups on a CU; 4-bit keys spill 11 of them for it
+// At d = 128 the bound of 128 registers keeps two workgroups on a CU; 4-bit keys spill 8 of them for it
 // (4/2-bit codes within 2 % of the fp64 scores' time at 1,000 to 65,536 rows, 16 x 131,072 rows in 3/3-bit
 // codes 732 us, 812 before).
 template <int D, int KB, bool SEQ, bool QS, bool STEP>
